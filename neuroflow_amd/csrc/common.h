@@ -85,6 +85,32 @@ __device__ __forceinline__ int32_t quant_i8_near(float a, float inv_s, uint64_t&
     return static_cast<int32_t>(r);
 }
 
+// Fixed-scale INT8 code (QuantiseActivation with scale_A, zp_A) by the
+// reciprocal, and whether it is certainly the reference's.  inv = fl(1 / s)
+// correctly rounded and, for s in [2^-120, 2^120] (the caller's condition),
+// normal; t = fl(a * inv) and q = fl(a / s) then each lie within
+// 2^-24 |a / s| (t: 2 * 2^-24) of a / s, so |t - q| <= 3 * 2^-24 |a / s|
+// < 2^-22 |t| (a subnormal product is below 2^-126 and gives r = q = 0).
+// |t - r| with r = rint(t) is exact (t and r within a factor 2, or r = 0).
+// If |t - r| < 0.5 - 2^-20 |t| (so |t| < 2^19), then |q - r| < 0.5:
+// round-half-away(q) == r, and the code is clamp(r + zp) with the
+// reference's wrapping add.  NaN / Inf elements give a NaN distance and are
+// rejected.
+__device__ __forceinline__ int32_t quant_i8_fixed_near(float a, float inv, int32_t zp, bool& bad) {
+    const float t = a * inv;
+    const float r = rintf(t);
+    const float lim = __builtin_fmaf(fabsf(t), -0x1p-20f, 0.5f);
+    bad = !(fabsf(t - r) < lim);
+    const int32_t ri = bad ? 0 : static_cast<int32_t>(r);
+    return clamp_i8(static_cast<int32_t>(static_cast<uint32_t>(ri) + static_cast<uint32_t>(zp)));
+}
+
+// The exact code of element e of x (kept out of line: the rare patch path).
+__device__ __attribute__((noinline)) uint32_t patch_fixed_code(uint32_t word, float v, int e, float s, int32_t zp) {
+    const uint32_t c = static_cast<uint32_t>(quant_i8_exact(v, s, zp)) & 0xFFu;
+    return (word & ~(0xFFu << (8 * e))) | (c << (8 * e));
+}
+
 // Pack four int8 codes (low byte first) into one dword: two v_perm_b32
 // select the low bytes (selector 0x0c zeroes a byte).
 __device__ __forceinline__ uint32_t pack4(int32_t a, int32_t b, int32_t c, int32_t d) {
@@ -178,6 +204,40 @@ __device__ __forceinline__ float fp8_value(float x, float inv) {
     const float xs = x * inv;
     const float v = fp8_value_of(xs);
     return __builtin_isnan(xs) ? xs : v;
+}
+
+// The clamped, pre-rounded value whose hardware E4M3 conversion is the byte
+// of fp8_quant: v_cvt_pk_fp8_f32 rounds to three mantissa bits (2^-9 steps
+// below 2^-6), ties to even, as e4m3_encode does, except that e4m3_encode
+// caps |xc| in (7.5 * 2^-9, 2^-6) at 7 * 2^-9 where the hardware rounds up
+// to 2^-6; clamping those to 7 * 2^-9 first makes the two agree.  NaN stays
+// NaN (the conversion then gives a NaN byte, of either sign).
+__device__ __forceinline__ float fp8_prerounded(float x, float inv) {
+    const float xs = x * inv;
+    const float xc = __builtin_amdgcn_fmed3f(xs, -448.0f, 448.0f);   // xs not NaN
+    const float sub = __builtin_amdgcn_fmed3f(xc, -7.0f * 0x1p-9f, 7.0f * 0x1p-9f);
+    const float v = fabsf(xc) < 0x1p-6f ? sub : xc;
+    return __builtin_isnan(xs) ? xs : v;
+}
+
+// Four E4M3 bytes of a lane's four values, low byte first.
+__device__ __forceinline__ uint32_t fp8_pack4(v4f x, float inv) {
+    int w = __builtin_amdgcn_cvt_pk_fp8_f32(fp8_prerounded(x[0], inv), fp8_prerounded(x[1], inv), 0, false);
+    w = __builtin_amdgcn_cvt_pk_fp8_f32(fp8_prerounded(x[2], inv), fp8_prerounded(x[3], inv), w, true);
+    return static_cast<uint32_t>(w);
+}
+
+// Eight E4M3 bytes (two dwords) as the bf16 operand of one K = 32 MFMA
+// (v_cvt_scalef32_pk_bf16_fp8, scale 1: every E4M3 value is exact in bf16).
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ v8bf fp8x8_to_bf16(int lo, int hi) {
+    const v4i o = {
+        __builtin_bit_cast(int, v2bf(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false))),
+        __builtin_bit_cast(int, v2bf(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true))),
+        __builtin_bit_cast(int, v2bf(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false))),
+        __builtin_bit_cast(int, v2bf(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true)))};
+    return __builtin_bit_cast(v8bf, o);
 }
 
 // bfloat16 bits of two E4M3 values held as fp32, low half first (one v_perm).

@@ -52,6 +52,7 @@ struct KernelPath {
     std::atomic<int> no_gemm{0};
     std::atomic<int> no_rows64{0};
     std::atomic<int> no_token_gemm{0};
+    std::atomic<int> token_rows{0};  // 0: the launcher's choice, else 16 or 64 rows per tile
     std::atomic<int> gemm_reg{0};
     std::atomic<int> gemm_tile{0};   // 0: the launcher's choice
     std::atomic<int> gemm_mfma{0};   // 0: the launcher's choice, else 16 or 32
@@ -68,13 +69,15 @@ inline bool aligned(const void* p, uintptr_t a) {
     return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0;
 }
 
-// Row-tile kernel eligibility for the given input mode.
-inline bool rows_ok(const RowsArgs& a, int in_mode) {
+// Row-tile kernel eligibility for the given input mode.  On fp32 input it
+// serves the layers whose weights it holds in registers (N <= 64, K up to 128
+// in INT8 and 64 in FP8); the one-pass kernel takes the others.
+inline bool rows_ok(const RowsArgs& a, int in_mode, bool fp8 = false) {
     if (a.K % 4 != 0 || a.N % 4 != 0) return false;
     if (in_mode == IN_CODES) {
         if (a.K > 1024 || !aligned(a.Aq, 4)) return false;
     } else {
-        if (a.K > 256 || !aligned(a.A, 16)) return false;
+        if (a.N > 64 || !rows_hoist_fits((a.K + 63) / 64, fp8) || !aligned(a.A, 16)) return false;
     }
     return aligned(a.W, 4) && aligned(a.C, 16);
 }
@@ -98,10 +101,14 @@ void launch_rows64(const RowsArgs& a, int act, hipStream_t st);
 // Its fixed-scale INT8 form (one scale_A / zp_A for every row, no activation).
 void launch_rows64_fixed(const RowsArgs& a, hipStream_t st);
 
-// The one-pass per-token INT8 layer for K = 128 / 256 / 512, N % 64 == 0
-// (token_gemm.hip): quantise into LDS, then the whole N range.
+// The one-pass layer for K <= 1024 (token_*.hip): quantise into LDS, then the
+// whole N range.
 bool token_gemm_ok(const RowsArgs& a);
-void launch_token_gemm(const RowsArgs& a, int act, hipStream_t st);
+// Whether it takes tiles of 16 rows (and 128-column chunks) instead of 64.
+bool token_small_tiles(const RowsArgs& a);
+void launch_token_i8(const RowsArgs& a, int act, hipStream_t st);
+void launch_token_i8_fixed(const RowsArgs& a, hipStream_t st);
+void launch_token_fp8(const RowsArgs& a, int act, hipStream_t st);
 
 // The tiled MFMA GEMM on INT8 codes for K a multiple of 64, K >= 128 (gemm.hip).
 bool gemm_ok(const RowsArgs& a);

@@ -512,6 +512,36 @@ static int kb_dot_for(int formula, int K) {
 
 static int formula_row(int K) { return K <= 4096 ? F_ROW_VNNI : F_ROW_SCALAR; }
 
+// Whether a layer on fp32 input takes the one-pass kernel (token_gemm_kernel.h)
+// rather than the row-tile kernel or the generic one.  The row-tile kernel
+// stays where it can run (weights in registers: 300000 x 64 -> 40 26.9 us
+// either way).
+static bool use_token_gemm(const RowsArgs& a, bool fp8) {
+    if (!token_gemm_ok(a) || path_flag(kernel_path().no_token_gemm)) return false;
+    return !rows_ok(a, IN_F32_TOKEN, fp8);
+}
+
+// Per-token INT8 shapes the tiled GEMM could also take (after a quantise
+// launch): whether that split is the faster form.  The one-pass kernel reads
+// all the weights once per row tile, the split form reads the activations
+// once and the codes per column block.  Measured on MI355X (us, one-pass /
+// split): K <= 256 one-pass throughout (12000 x 256 -> 1024 18.1 / 20.1, 65536
+// x 192 -> 2048 127 / 161) but for wide rows of part lines (20000 x 256 ->
+// 1000 33.6 / 28.5); larger K at 16-row tiles one-pass (1500 x 320 -> 512 8.8 /
+// 9.8, 3000 x 512 -> 256 10.2 / 10.9); at 64-row tiles split (12000 x 384 ->
+// 1024 29 / 27, 8192 x 512 -> 1024 22 / 17) until there are enough row tiles
+// (20000 x 512 -> 256 19.7 / 22.2, 32768 x 384 -> 2048 83 / 102), and split again
+// at K = 512 with wide N, where the persistent GEMM runs (65536 x 512 -> 768
+// 85 / 73, -> 2048 183 / 145).
+static bool split_faster(const RowsArgs& a) {
+    if (a.K > 512) return true;
+    if (a.K <= 256) return a.K > 192 && a.N > 512 && a.N % 32 != 0 && a.M < 32768 && !token_small_tiles(a);
+    if (token_small_tiles(a)) return false;
+    if (a.M < 16384) return true;
+    if (a.N <= 256) return false;
+    return a.M < 32768 || (a.K == 512 && a.N > 512 && a.N % 32 == 0);
+}
+
 // Fixed-scale int8 path shared by LinearForward / rows / batched.
 static int int8_fixed_path(const nflow_int8_linear_params* p, int64_t rows, const float* A, float* C,
                            int formula, hipStream_t st, const char* what) {
@@ -532,6 +562,10 @@ static int int8_fixed_path(const nflow_int8_linear_params* p, int64_t rows, cons
     a.C = C;
     if (rows64_ok(a) && !path_flag(kernel_path().no_rows64)) {
         launch_rows64_fixed(a, st);
+        return check_launch(what);
+    }
+    if (use_token_gemm(a, false)) {
+        launch_token_i8_fixed(a, st);
         return check_launch(what);
     }
     if (rows_ok(a, IN_F32_FIXED)) {
@@ -579,6 +613,7 @@ int nflow_debug_set_kernel_path(const char* name, int value, int* previous) {
     std::atomic<int>* f = n == "no_gemm" ? &k.no_gemm
                         : n == "no_rows64" ? &k.no_rows64
                         : n == "no_token_gemm" ? &k.no_token_gemm
+                        : n == "token_rows" ? &k.token_rows
                         : n == "gemm_reg" ? &k.gemm_reg
                         : n == "gemm_tile" ? &k.gemm_tile
                         : n == "gemm_mfma" ? &k.gemm_mfma
@@ -734,6 +769,33 @@ struct FixedWs {
     const char* what;
 };
 
+// The split path's workspace: codes, then (with no scale_A_out) M scales, then
+// M row code sums when zero points may be nonzero and N weight-row byte sums
+// when the formula takes a caller's sum_W (both for the tiled GEMM only).
+static size_t split_sums(const RowsArgs& a, bool wide) {
+    const bool want_sums = wide && a.zpW;
+    const bool want_colsum = wide && a.formula == F_ROW_VNNI && a.sumW;
+    return (want_sums ? static_cast<size_t>(a.M) : 0) + (want_colsum ? a.N : 0);
+}
+static size_t noalloc_need(const RowsArgs& a, bool wide) {
+    const size_t codes16 = ((static_cast<size_t>(a.M) * a.K + 15) / 16) * 16;
+    return codes16 + (a.scale_out ? 0 : static_cast<size_t>(a.M) * sizeof(float)) +
+           split_sums(a, wide) * sizeof(int32_t);
+}
+// Shapes the no-allocation entry point documents as too large for its
+// scratch: those whose codes the split path holds there, also where the
+// one-pass kernel, which needs none, runs them (K = 128, 256 and 512 with N a
+// multiple of 64, and aligned K <= 256 the tiled GEMM cannot take, are never
+// refused).
+static bool noalloc_refuses(const RowsArgs& a, bool wide, size_t cap) {
+    const bool one_pass = (a.K == 128 || a.K == 256 || a.K == 512) && a.N % 64 == 0 && aligned(a.A, 16) &&
+                          aligned(a.C, 16) && aligned(a.W, 16);
+    const bool narrow = !wide && a.K <= 256 && a.K % 4 == 0 && a.N % 4 == 0 && aligned(a.A, 16) &&
+                        aligned(a.W, 4) && aligned(a.C, 16);
+    if (one_pass || narrow) return false;
+    return noalloc_need(a, wide) > cap;
+}
+
 static int int8_per_token(const nflow_int8_linear_params* p, int64_t M, const float* A,
                           const float* R, float* C, float* scale_A_out, int activation,
                           const nflow_x2_quant* xq, void* stream, const FixedWs* fixed = nullptr) {
@@ -773,15 +835,14 @@ static int int8_per_token(const nflow_int8_linear_params* p, int64_t M, const fl
         if (post) hipLaunchKernelGGL(k_fno_post, dim3(grid_for(M, 1, 16)), dim3(256), 0, st, C, R, a, activation);
         return check_launch("linear_forward_per_token");
     };
-    // K = 128 .. 512: the one-pass kernel (quantise into LDS, then all of N).
-    if (token_gemm_ok(a) && !path_flag(kernel_path().no_token_gemm)) {
-        launch_token_gemm(a, act_x2, st);
-        return finish();
-    }
     // Wide K: quantise into a workspace, then the tiled GEMM (below).
     RowsArgs g = a;
     g.Aq = nullptr;  // the codes go to the workspace, which is 256-byte aligned
     const bool wide = use_gemm(g);
+    if (use_token_gemm(a, false) && !(wide && split_faster(a)) && !(fixed && noalloc_refuses(a, wide, fixed->cap))) {
+        launch_token_i8(a, act_x2, st);
+        return finish();
+    }
     if (!wide && rows_ok(a, IN_F32_TOKEN)) {
         launch_rows<false, IN_F32_TOKEN, OUT_EPI>(a, act_x2, st);
         return finish();
@@ -793,13 +854,12 @@ static int int8_per_token(const nflow_int8_linear_params* p, int64_t M, const fl
     const size_t codes = static_cast<size_t>(M) * a.K;
     const bool want_sums = wide && a.zpW;
     const bool want_colsum = wide && a.formula == F_ROW_VNNI && a.sumW;
-    const size_t n_sums = (want_sums ? static_cast<size_t>(M) : 0) + (want_colsum ? a.N : 0);
+    const size_t n_sums = split_sums(a, wide);
     const size_t codes16 = ((codes + 15) / 16) * 16;
     if (fixed) {
         // Codes, then (with no scale_A_out) M scales, then the sums; every
         // region is written by the quantise launch before the product reads it.
-        const size_t need = codes16 + (scale_A_out ? 0 : static_cast<size_t>(M) * sizeof(float)) +
-                            n_sums * sizeof(int32_t);
+        const size_t need = noalloc_need(a, wide);
         if (need > fixed->cap)
             return set_error(NFLOW_INVALID_ARG, std::string(fixed->what) + ": this shape needs " +
                                                     std::to_string(need) + " bytes of scratch, more than the " +
@@ -1023,7 +1083,11 @@ static int fp8_per_token(const nflow_fp8_linear_params* p, int64_t M, const floa
         if (post) hipLaunchKernelGGL(k_fno_post, dim3(grid_for(M, 1, 16)), dim3(256), 0, st, C, R, a, activation);
         return check_launch("fp8_linear_forward_per_token");
     };
-    if (rows_ok(a, IN_F32_TOKEN)) {
+    if (use_token_gemm(a, true)) {
+        launch_token_fp8(a, act_x2, st);
+        return finish();
+    }
+    if (rows_ok(a, IN_F32_TOKEN, true)) {
         launch_rows<true, IN_F32_TOKEN, OUT_EPI>(a, act_x2, st);
         return finish();
     }

@@ -97,32 +97,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const void* base, in
         static_cast<int>(left) * row_bytes, 0x00020000);
 }
 
-// Fixed-scale INT8 code (QuantiseActivation with scale_A, zp_A) by the
-// reciprocal, and whether it is certainly the reference's.  inv = fl(1 / s)
-// correctly rounded and, for s in [2^-120, 2^120] (the caller's condition),
-// normal; t = fl(a * inv) and q = fl(a / s) then each lie within
-// 2^-24 |a / s| (t: 2 * 2^-24) of a / s, so |t - q| <= 3 * 2^-24 |a / s|
-// < 2^-22 |t| (a subnormal product is below 2^-126 and gives r = q = 0).
-// |t - r| with r = rint(t) is exact (t and r within a factor 2, or r = 0).
-// If |t - r| < 0.5 - 2^-20 |t| (so |t| < 2^19), then |q - r| < 0.5:
-// round-half-away(q) == r, and the code is clamp(r + zp) with the
-// reference's wrapping add.  NaN / Inf elements give a NaN distance and are
-// rejected.
-__device__ __forceinline__ int32_t quant_i8_fixed_near(float a, float inv, int32_t zp, bool& bad) {
-    const float t = a * inv;
-    const float r = rintf(t);
-    const float lim = __builtin_fmaf(fabsf(t), -0x1p-20f, 0.5f);
-    bad = !(fabsf(t - r) < lim);
-    const int32_t ri = bad ? 0 : static_cast<int32_t>(r);
-    return clamp_i8(static_cast<int32_t>(static_cast<uint32_t>(ri) + static_cast<uint32_t>(zp)));
-}
-
-// The exact code of element e of x (kept out of line: the rare patch path).
-__device__ __attribute__((noinline)) uint32_t patch_fixed_code(uint32_t word, float v, int e, float s, int32_t zp) {
-    const uint32_t c = static_cast<uint32_t>(quant_i8_exact(v, s, zp)) & 0xFFu;
-    return (word & ~(0xFFu << (8 * e))) | (c << (8 * e));
-}
-
 // A row takes the exact path when its fast absmax is NaN (a signalling NaN
 // in the row) or, for INT8, when amax / 127 would be subnormal (t may then
 // leave the int8 range).

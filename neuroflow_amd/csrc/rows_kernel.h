@@ -58,8 +58,6 @@ __device__ __forceinline__ void stream_store(T v, T* p) {
 #endif
 }
 
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-
 enum InMode { IN_F32_TOKEN = 0, IN_F32_FIXED = 1, IN_CODES = 2 };
 enum OutMode { OUT_EPI = 0, OUT_RAW = 1 };
 

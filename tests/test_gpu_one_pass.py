@@ -1,0 +1,140 @@
+"""The one-pass layer kernel (quantise into LDS, then the whole N range) at the
+sizes where it can go wrong, against the oracle: K and N off every tile
+(K % 64, K % 4, N % 64, N % 4, K below a wave's float4s), row counts around
+the 16- and 64-row tiles, buffers aligned to 4 bytes only, the column chunks
+shared over blocks, per-token INT8, fixed-scale INT8 (both formulas, with the
+row form's dropped K tail) and FP8, on either tile height.
+
+INT8 outputs must equal the oracle's bits (codes, accumulators and dequantise
+are exact); FP8 is held to K * 2^-24 * sum|terms| (fp32 accumulation of exact
+products) plus the three roundings of the dequantise."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from neuroflow_amd import _lib
+from neuroflow_amd import quant as Q
+from neuroflow_amd import workloads as WL
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# (M, K, N): tile edges and remainders of the 16 / 64-row tiles, the 64-wide
+# K blocks (template sizes 64, 128, 256, 512, 1024) and the 128 / 256-column
+# chunks; the last ones cross the 16-row line and share chunks over blocks.
+SHAPES = [(1, 4, 4), (3, 5, 7), (17, 64, 65), (63, 67, 127), (64, 128, 128), (65, 130, 129), (16, 192, 256),
+          (129, 255, 300), (40, 257, 64), (70, 320, 200), (33, 511, 96), (15, 512, 257), (48, 513, 66),
+          (31, 1000, 130), (18, 1023, 33), (20000, 101, 128), (9000, 256, 513), (300, 100, 1030)]
+
+
+@pytest.fixture(params=[0, 16, 64], ids=["auto", "rows16", "rows64"])
+def tile_rows(request):
+    prev = ctypes.c_int(0)
+    L = _lib.lib()
+    _lib.check(L.nflow_debug_set_kernel_path(b"token_rows", request.param, ctypes.byref(prev)), "path")
+    yield request.param
+    _lib.check(L.nflow_debug_set_kernel_path(b"token_rows", prev.value, None), "path")
+
+
+def _cu(a, off):
+    """A device copy that starts `off` elements past a 256-byte boundary."""
+    a = np.ascontiguousarray(a)
+    buf = torch.empty(a.size + off, dtype=torch.from_numpy(a[:0].reshape(-1)).dtype, device="cuda")
+    out = buf[off:].view(a.shape)
+    out.copy_(torch.from_numpy(a))
+    return out
+
+
+def _guarded(M, N, off):
+    """An (M, N) output `off` floats past a boundary, with guards around it."""
+    buf = torch.full((M * N + 64 + off,), 7.0, dtype=torch.float32, device="cuda")
+    return buf, buf[off:off + M * N].view(M, N)
+
+
+def _guards_kept(buf, M, N, off):
+    return bool((buf[:off] == 7.0).all()) and bool((buf[off + M * N:] == 7.0).all())
+
+
+def _rows(M):
+    return np.arange(M) if M <= 512 else np.unique(np.concatenate([np.arange(70), np.arange(M - 70, M),
+                                                                   np.arange(0, M, 89)]))
+
+
+def _int8(N, K, sid):
+    W = WL.uniform(sid, (N, K), -0.125, 0.125)
+    s = O.per_channel_scales(W, 127.0)
+    zps = WL.uniform(sid + 1, (N,), -6, 6).astype(np.int32)
+    q, sw = O.quantise_weight_2d(W, s, zps)
+    return q, s, zps, sw, WL.uniform(sid + 2, (N,), -0.1, 0.1)
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+@pytest.mark.parametrize("zp", [False, True])
+def test_per_token_int8(gpu, tile_rows, M, K, N, zp):
+    off = (M + K + N) % 3
+    q, s, zps, sw, b = _int8(N, K, 800)
+    A = WL.normal(803, (M, K))
+    A[M // 2] = 0.0
+    p = Q.Int8LinearParams(_cu(q, off), _cu(s, 0), _cu(zps, 0) if zp else None, _cu(b, 0),
+                           sum_W_per_row=_cu(sw, 0) if zp else None)
+    buf, out = _guarded(M, N, off)
+    y, sc = Q.linear_forward_per_token(p, _cu(A, off), "relu", out=out, return_scales=True)
+    rows = _rows(M)
+    want, s_want = O.layer_per_token_i8(A[rows], q, s, zps if zp else None, b, sw if zp else None, 1)
+    assert np.array_equal(sc.cpu().numpy()[rows].view(np.uint32), s_want.view(np.uint32))
+    assert np.array_equal(y.cpu().numpy()[rows].view(np.uint32), want.view(np.uint32))
+    assert _guards_kept(buf, M, N, off)
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+@pytest.mark.parametrize("form", ["rows", "batched"])
+def test_fixed_int8(gpu, tile_rows, M, K, N, form):
+    off = (M + K + N) % 3
+    q, s, zps, sw, b = _int8(N, K, 810)
+    A = WL.normal(813, (M, K))
+    A.reshape(-1)[:min(M * K, 8)] = np.array([np.nan, np.inf, -np.inf, 3e9, -3e9, 1e-40, -0.0, 0.05],
+                                             np.float32)[:min(M * K, 8)]
+    p = Q.Int8LinearParams(_cu(q, off), _cu(s, 0), _cu(zps, 0), _cu(b, 0), 0.02, 5,
+                           _cu(sw, 0) if form == "batched" else None)
+    fn, ref = ((Q.linear_forward_batched, O.linear_forward_batched) if form == "batched"
+               else (Q.linear_forward, O.linear_forward_rows))
+    y = fn(p, _cu(A, off)).cpu().numpy()
+    rows = _rows(M)
+    rc, want = ref(A[rows], q, s, zps, b, 0.02, 5, sw if form == "batched" else None)
+    assert rc == 0
+    assert np.array_equal(y[rows].view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+def test_fp8(gpu, tile_rows, M, K, N):
+    off = (M + K + N) % 3
+    A = (2.0 * WL.normal(820, (M, K))).astype(np.float32)
+    A = np.where(WL.uniform(821, (M, K)) < 0.02, 20.0 * A, A).astype(np.float32)
+    A[M // 2] = 0.0
+    if M > 8:
+        A[1, -1] = np.nan
+        A[2, 0] = np.inf
+        A[3] = 1e-40          # a subnormal row scale: its reciprocal is infinite
+        A[3, 0] = 0.0
+        A[4, :] = (np.arange(K) % 64 - 32) * 2.0 ** -9     # around the subnormal cap of the format
+        A[4, 0] = 448.0
+    W = WL.uniform(822, (N, K), -0.125, 0.125)
+    b = WL.uniform(823, (N,), -0.125, 0.125)
+    qw, sw = O.quantise_weight_fp8(W)
+    p = Q.Fp8LinearParams(_cu(qw, off), _cu(sw, 0), _cu(b, 0))
+    buf, out = _guarded(M, N, off)
+    y, sc = Q.fp8_linear_forward_per_token(p, _cu(A, off), "none", out=out, return_scales=True)
+    rows = _rows(M)
+    qa, sa = O.quantise_per_token_fp8(A[rows])
+    got = y.cpu().numpy()[rows]
+    assert np.array_equal(sc.cpu().numpy()[rows].view(np.uint32), sa.view(np.uint32))
+    want = O.layer_fp8_exact(qa, sa, qw, sw, b, 0)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    fin = np.isfinite(want).all(axis=1)
+    terms = (np.abs(O.e4m3_decode(qa[fin])) * sa[fin, None]).astype(np.float64) @ \
+        (np.abs(O.e4m3_decode(qw)) * sw[:, None]).astype(np.float64).T
+    bound = (K + 3) * 2.0 ** -24 * (terms + np.abs(b)[None, :]) + 1e-38
+    assert np.all(np.abs(got[fin].astype(np.float64) - want[fin]) <= bound)
+    assert _guards_kept(buf, M, N, off)
