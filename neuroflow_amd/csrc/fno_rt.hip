@@ -18,22 +18,10 @@
 #include "gelu_exact.h"
 #include "launch.h"
 #include "rows64_kernel.h"
+#include "fno_dev.h"
 #include "snap.h"
 
 namespace nfq {
-
-__device__ __forceinline__ float rt_activate(float y, int act) {
-    if (act == RT_ACT_RELU) return y < 0.0f ? 0.0f : y;  // fno.cpp:37-40
-    if (act == RT_ACT_GELU) return gelu_fast<kGeluRefine>(y);
-    return y;
-}
-
-// LDS written by some lanes of a wave, read by others after this point.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Logical block of this launch when blocks are dealt round-robin to the 8
 // XCDs: each XCD takes a contiguous range of logical blocks, so the blocks
@@ -44,14 +32,6 @@ __device__ __forceinline__ int64_t xcd_block(int64_t nlogical) {
     const int64_t b = static_cast<int64_t>(blockIdx.x);
     const int64_t logical = (b % 8) * per + b / 8;
     return logical < nlogical ? logical : -1;
-}
-
-// ---------------------------------------------------------------------------
-// fp32 Linear (fno.cpp:69-79) in the reference build's summation order: the
-// first k - k % 8 products rounded and added one by one, the rest fused.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ float lin_step(float acc, float x, float w, bool plain) {
-    return plain ? acc + x * w : __builtin_fmaf(x, w, acc);
 }
 
 // k == 64, n >= 16: one wave per 4 output rows; lane j holds column j of W
@@ -245,6 +225,103 @@ __global__ __launch_bounds__(256) void k_linear_k1(LinArgs a) {
     }
 }
 
+// Any k whose tiles fit the LDS, any n: a block stages CW columns of W
+// (transposed) and its rows' inputs in LDS; lane c of a row group holds
+// column c of kLinRows rows, so a step reads one weight and kLinRows
+// broadcast inputs per kLinRows outputs.  The one-thread-per-output form
+// below reads both operands of every product from the cache (262144 x 32 ->
+// 32: 473 us).  Row r of the launch is output row r; its input row and
+// validity follow LinArgs.
+constexpr int kLinRows = 8;
+constexpr int lin_block_rows(int cw) { return 4 * (64 / cw) * kLinRows; }
+inline size_t lin_block_lds(int k, int cw) {
+    const size_t ks = (static_cast<size_t>(k) + 3) / 4 * 4;
+    return (ks * cw + lin_block_rows(cw) * (ks + 4)) * sizeof(float);
+}
+
+template <int CW>
+__global__ __launch_bounds__(256) void k_linear_block(LinArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float lsm[];
+    constexpr int G = 64 / CW, BR = lin_block_rows(CW);
+    const int k = a.k, n = a.n, kplain = k - k % 8, ks = (k + 3) / 4 * 4, xst = ks + 4;
+    float* wt = lsm;                    // [k][CW]
+    float* xs = lsm + ks * CW;          // [BR][xst]
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int col = lane % CW, grp = lane / CW;
+    const int64_t rows = a.samples * a.rows_out;
+    const bool whole = a.rows_in == a.rows_out && a.rows_valid == a.rows_out;
+    for (int cc = 0; cc < n; cc += CW) {
+        __syncthreads();
+        for (int i = threadIdx.x; i < CW * k; i += 256) {
+            const int c = i / k, p = i - c * k;
+            wt[p * CW + c] = cc + c < n ? a.W[static_cast<int64_t>(cc + c) * k + p] : 0.0f;
+        }
+        const int j = cc + col;
+        const float bj = j < n && a.b ? a.b[j] : 0.0f;
+        for (int64_t r0 = static_cast<int64_t>(blockIdx.x) * BR; r0 < rows; r0 += static_cast<int64_t>(gridDim.x) * BR) {
+            const int nr = rows - r0 < BR ? static_cast<int>(rows - r0) : BR;
+            __syncthreads();
+            if (whole && k % 4 == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0) {
+                const int kq = k / 4;
+                const v4f* x4 = reinterpret_cast<const v4f*>(a.x + r0 * k);
+                for (int i = threadIdx.x; i < nr * kq; i += 256) {
+                    const int t = i / kq;
+                    *reinterpret_cast<v4f*>(xs + t * xst + 4 * (i - t * kq)) = x4[i];
+                }
+            } else {
+                for (int i = threadIdx.x; i < nr * k; i += 256) {
+                    const int t = i / k;
+                    int64_t src = r0 + t;
+                    bool ok = true;
+                    if (!whole) {
+                        const int64_t s = src / a.rows_out;
+                        const int q = static_cast<int>(src - s * a.rows_out);
+                        ok = q < a.rows_valid;
+                        src = s * a.rows_in + q;
+                    }
+                    xs[t * xst + (i - t * k)] = ok ? a.x[src * k + (i - t * k)] : 0.0f;
+                }
+            }
+            __syncthreads();
+            // Row m of the lane: wid * (BR / 4) + m * G + grp.
+            const float* xr = xs + (wid * (BR / 4) + grp) * xst;
+            float acc[kLinRows];
+#pragma unroll
+            for (int m = 0; m < kLinRows; ++m) acc[m] = bj;
+            for (int p = 0; p < kplain; p += 4) {
+                float w[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) w[e] = wt[(p + e) * CW + col];
+#pragma unroll
+                for (int m = 0; m < kLinRows; ++m) {
+                    const v4f x = *reinterpret_cast<const v4f*>(xr + m * G * xst + p);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[m] = acc[m] + x[e] * w[e];
+                }
+            }
+            for (int p = kplain; p < k; ++p) {
+                const float w = wt[p * CW + col];
+#pragma unroll
+                for (int m = 0; m < kLinRows; ++m) acc[m] = __builtin_fmaf(xr[m * G * xst + p], w, acc[m]);
+            }
+#pragma unroll
+            for (int m = 0; m < kLinRows; ++m) {
+                const int t = wid * (BR / 4) + m * G + grp;
+                if (t >= nr || j >= n) continue;
+                const int64_t r = r0 + t;
+                const bool valid = whole || static_cast<int>(r % a.rows_out) < a.rows_valid;
+                a.y[r * n + j] = valid ? rt_activate(acc[m], a.act) : 0.0f;
+            }
+        }
+    }
+}
+
+template <int CW>
+static void launch_linear_block(const LinArgs& a, int64_t rows, hipStream_t st) {
+    hipLaunchKernelGGL(k_linear_block<CW>, dim3(grid_for(rows, lin_block_rows(CW), 8)), dim3(256),
+                       lin_block_lds(a.k, CW), st, a);
+}
+
 // Any shape: one thread per output.
 __global__ __launch_bounds__(256) void k_linear_flat(LinArgs a) {
     const int k = a.k, n = a.n, kplain = k - k % 8;
@@ -294,82 +371,6 @@ __global__ __launch_bounds__(256) void k_linear_flat(LinArgs a) {
 // ---------------------------------------------------------------------------
 // Layout change and the layer tail, on 64-point x 64-channel tiles.
 // ---------------------------------------------------------------------------
-struct Tile {
-    int64_t s;
-    int t0, c0;
-};
-
-// Tile `id` of TT tokens x 64 channels.
-template <int TT>
-__device__ __forceinline__ bool tile_of(int64_t id, int64_t samples, int n, int w, Tile& tl) {
-    const int tt = (n + TT - 1) / TT, tc = (w + 63) / 64;
-    const int64_t per_sample = static_cast<int64_t>(tt) * tc;
-    if (id >= samples * per_sample) return false;
-    tl.s = id / per_sample;
-    const int rem = static_cast<int>(id % per_sample);
-    tl.t0 = (rem / tc) * TT;
-    tl.c0 = (rem % tc) * 64;
-    return true;
-}
-
-// fno.cpp:579-606 with the exponent e = int(std::round(log2|v| * 8) / 8)
-// read off the step points of the reference's libm (thr: the smallest float
-// of each exponent from -5 to 9, computed on the host with that libm):
-// e = -6 + #{thr <= |v|} for 2^-6 <= |v| <= FLT_MAX, taken from |v|'s binade
-// and one compare (snap.h; thr in LDS); NaN and Inf give ldexp(1, INT_MIN)
-// = 0; 2^e for e >= 9 is capped at 448.
-__device__ __forceinline__ float log2_snap(float x, float s, const float* thr) {
-    const float v = x / s;
-    const float av = fabsf(v);
-    const float sign = v < 0.0f ? -1.0f : 1.0f;
-    float qv;
-    if (av < 0.015625f) {
-        qv = av;
-    } else if (!(av <= 0x1.fffffep+127f)) {
-        qv = 0.0f;
-    } else {
-        const int e = snap_exponent_binade(av, thr);
-        qv = e >= 9 ? 448.0f : __builtin_bit_cast(float, static_cast<uint32_t>(127 + e) << 23);
-    }
-    const float clamped = (448.0f < qv) ? 448.0f : qv;
-    return (sign * clamped) * s;
-}
-
-// x2_fake_quant with the per-tensor scale's reciprocal inv = fl(1 / s)
-// computed once (inv_ok: inv a normal float).  t = v * inv is within
-// 1.5 * 2^-23 |t| of the quotient fl(v / s), so while |t| is farther than
-// 2^-20 |t| from the nearest half-integer, rint(t) equals round(fl(v / s))
-// (the two rounding rules differ only on ties) and the rest of the
-// fake-quant follows unchanged; otherwise (near a tie, |t| >= 2^22, NaN,
-// Inf) the exact division.
-__device__ __forceinline__ float x2_fake_quant_inv(float v, float s, float inv, bool inv_ok, float zpf) {
-    const float t = v * inv;
-    const float at = fabsf(t);
-    const float dist = fabsf(__builtin_amdgcn_fractf(at) - 0.5f);
-    if (!(inv_ok && dist > __builtin_fmaf(at, 0x1p-20f, 0x1p-40f))) return x2_fake_quant(v, s, zpf);
-    float q = rintf(t) + zpf;
-    q = q < -128.0f ? -128.0f : q;
-    q = q > 127.0f ? 127.0f : q;
-    return (q - zpf) * s;
-}
-
-// The reciprocal of a per-tensor scale and whether it is a normal float.
-struct ScaleInv {
-    float inv;
-    bool ok;
-};
-__device__ __forceinline__ ScaleInv scale_inv(float s) {
-    const float inv = 1.0f / s;
-    const float a = fabsf(inv);
-    return {inv, a >= 0x1p-126f && a <= 0x1.fffffep+127f};
-}
-
-// Copies a step table into LDS; every thread of the block must call it.
-__device__ __forceinline__ void stage_steps(float* steps, const float* thr) {
-    if (threadIdx.x < 15) steps[threadIdx.x] = thr[threadIdx.x];
-    __syncthreads();
-}
-
 // The input fake-quant's form FQ (0 off, 1 per tensor, 3 log2 snap) is a
 // template parameter and each thread's offsets are its fixed offset plus q
 // times a per-launch stride, as in the layer tail below; thread x holds
@@ -1217,21 +1218,6 @@ __global__ __launch_bounds__(64 * WPB) void k_cfft_cols(ColArgs a, int64_t nlogi
 // offset plus q times a per-launch stride.  Each thread's elements of a tile
 // are loaded together (every load of a phase issued before the first is
 // waited for); the stores follow all of the phase's results.
-template <int KIND, int ACT, int FQN>
-__device__ __forceinline__ float post_element(float x1, float x2, const PostArgs& a, const ScaleInv& inv_x2,
-                                              const ScaleInv& inv_next, const float* thr_x2,
-                                              const float* thr_next, float pscale, float pzp) {
-    if constexpr (KIND == 1) x2 = x2_fake_quant_inv(x2, a.scale, inv_x2.inv, inv_x2.ok, a.zpf);
-    else if constexpr (KIND == 2) x2 = x2_fake_quant(x2, pscale, pzp);
-    else if constexpr (KIND == 3) x2 = log2_snap(x2, a.scale, thr_x2);
-    float y = x1 + x2;
-    if constexpr (ACT == RT_ACT_RELU) y = y < 0.0f ? 0.0f : y;   // fno.cpp:37-40
-    else if constexpr (ACT == RT_ACT_GELU) y = gelu_fast<kGeluRefine>(y);
-    if constexpr (FQN == 1) y = x2_fake_quant_inv(y, a.fq_next.scale, inv_next.inv, inv_next.ok, a.fq_next.zpf);
-    else if constexpr (FQN == 3) y = log2_snap(y, a.fq_next.scale, thr_next);
-    return y;
-}
-
 template <int TT, int KIND, int ACT, int FQN>
 __global__ __launch_bounds__(256) void k_post_rt(PostArgs a) {
     constexpr int PER = TT * 64 / 256;   // elements per thread and tile
@@ -1663,14 +1649,13 @@ hipError_t launch_linear_ref(const LinArgs& a, hipStream_t st) {
     } else if (a.k == 1 && a.rows_in == a.rows_out && a.rows_valid == a.rows_out && a.n >= 4 && a.n <= 1024 &&
                (a.n & (a.n - 1)) == 0 && aligned(a.y, 16)) {
         hipLaunchKernelGGL(k_linear_k1, dim3(grid_for(rows * (a.n / 4), 256, 8)), dim3(256), 0, st, a);
+    } else if (lin_block_lds(a.k, a.n > 32 ? 64 : 32) <= 64 * 1024) {
+        if (a.n > 32) launch_linear_block<64>(a, rows, st);
+        else launch_linear_block<32>(a, rows, st);
     } else {
         hipLaunchKernelGGL(k_linear_flat, dim3(grid_for(rows * a.n, 256, 8)), dim3(256), 0, st, a);
     }
     return hipGetLastError();
-}
-
-static int64_t tile_count(int64_t samples, int n, int w, int tt) {
-    return samples * ((n + tt - 1) / tt) * static_cast<int64_t>((w + 63) / 64);
 }
 
 // Tiles of 64 tokens, or of 8 when 64-token tiles would give fewer than two
@@ -2026,7 +2011,9 @@ hipError_t launch_layer_tail(const LayerTailArgs& a, hipStream_t st) {
 
 // The fp32 local linear + tail: as layer_tail_ok, for a 64 x 64 fp32 layer
 // whose rows are read as 16-byte vectors.
-bool linear_tail_ok(const PostArgs& p, const float* W) { return layer_tail_ok(p, 64, 64) && aligned(W, 16); }
+bool linear_tail_ok(const PostArgs& p, const float* W) {
+    return p.w == 64 ? layer_tail_ok(p, 64, 64) && aligned(W, 16) : linear_tail_w_ok(p, W);
+}
 
 template <int KIND, int ACT>
 static void launch_linear_tail_fqn(const PostArgs& a, const float* W, const float* b, unsigned grid, hipStream_t st) {
@@ -2042,6 +2029,7 @@ static void launch_linear_tail_act(const PostArgs& a, const float* W, const floa
 
 hipError_t launch_linear_tail(const PostArgs& a, const float* W, const float* b, hipStream_t st) {
     if (a.samples <= 0) return hipSuccess;
+    if (a.w != 64) return launch_linear_tail_w(a, W, b, st);
     const unsigned grid = grid_for(tile_count(a.samples, a.n, a.w, 32), 1, 8);
     switch (a.kind) {
         case 1: launch_linear_tail_act<1>(a, W, b, grid, st); break;
@@ -2056,6 +2044,7 @@ hipError_t launch_linear_tail(const PostArgs& a, const float* W, const float* b,
 // whole 32-token tiles, at least two tiles per CU, the fake-quant forms off /
 // per tensor / log2 snap, 16-byte aligned h rows and proj_q weight.
 bool proj_tail_ok(const ProjArgs& p) {
+    if (p.w != 64) return proj_tail_w_ok(p);
     const auto fq_ok = [](const FakeQuant& f) { return f.on == 0 || f.on == 1 || f.on == 3; };
     return !path_flag(kernel_path().no_layer_tail) && p.w == 64 && p.out_ch == 1 && p.n > 0 && p.n % 32 == 0 &&
            p.rows_in >= p.n && tile_count(p.samples, p.n, 64, 32) >= 2 * static_cast<int64_t>(num_cus()) &&
@@ -2079,6 +2068,7 @@ static void launch_proj_tail_fqq(const ProjArgs& a, unsigned grid, hipStream_t s
 
 hipError_t launch_proj_tail(const ProjArgs& a, hipStream_t st) {
     if (a.samples <= 0) return hipSuccess;
+    if (a.w != 64) return launch_proj_tail_w(a, st);
     const unsigned grid = grid_for(tile_count(a.samples, a.n, 64, 32), 1, 8);
     if (a.act == RT_ACT_GELU) launch_proj_tail_fqq<RT_ACT_GELU>(a, grid, st);
     else if (a.act == RT_ACT_RELU) launch_proj_tail_fqq<RT_ACT_RELU>(a, grid, st);
