@@ -105,12 +105,6 @@ __device__ __forceinline__ int32_t quant_i8_fixed_near(float a, float inv, int32
     return clamp_i8(static_cast<int32_t>(static_cast<uint32_t>(ri) + static_cast<uint32_t>(zp)));
 }
 
-// The exact code of element e of x (kept out of line: the rare patch path).
-__device__ __attribute__((noinline)) uint32_t patch_fixed_code(uint32_t word, float v, int e, float s, int32_t zp) {
-    const uint32_t c = static_cast<uint32_t>(quant_i8_exact(v, s, zp)) & 0xFFu;
-    return (word & ~(0xFFu << (8 * e))) | (c << (8 * e));
-}
-
 // Pack four int8 codes (low byte first) into one dword: two v_perm_b32
 // select the low bytes (selector 0x0c zeroes a byte).
 __device__ __forceinline__ uint32_t pack4(int32_t a, int32_t b, int32_t c, int32_t d) {
@@ -119,6 +113,31 @@ __device__ __forceinline__ uint32_t pack4(int32_t a, int32_t b, int32_t c, int32
     const uint32_t hi = __builtin_amdgcn_perm(static_cast<uint32_t>(d), static_cast<uint32_t>(c),
                                               0x04000c0cu);
     return lo | hi;
+}
+
+// The exact code of element e of x (kept out of line: the rare patch path).
+__device__ __attribute__((noinline)) uint32_t patch_fixed_code(uint32_t word, float v, int e, float s, int32_t zp) {
+    const uint32_t c = static_cast<uint32_t>(quant_i8_exact(v, s, zp)) & 0xFFu;
+    return (word & ~(0xFFu << (8 * e))) | (c << (8 * e));
+}
+
+// The four codes of x with one scale: fast = the reciprocal path holds for s
+// (inv = fl(1 / s) normal); elements it is not certain of are redone exactly.
+__device__ __forceinline__ uint32_t quant_i8_fixed4(v4f x, float s, float inv, int32_t zp, bool fast) {
+    int32_t c[4];
+    bool any_bad = !fast;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        bool bad;
+        c[e] = quant_i8_fixed_near(x[e], inv, zp, bad);
+        any_bad |= bad;
+    }
+    uint32_t v = pack4(c[0], c[1], c[2], c[3]);
+    if (any_bad) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v = patch_fixed_code(v, x[e], e, s, zp);
+    }
+    return v;
 }
 
 // DPP row moves (16-lane rows): the lane pattern CTRL of v within each row.
@@ -210,20 +229,30 @@ __device__ __forceinline__ float fp8_value(float x, float inv) {
 // of fp8_quant: v_cvt_pk_fp8_f32 rounds to three mantissa bits (2^-9 steps
 // below 2^-6), ties to even, as e4m3_encode does, except that e4m3_encode
 // caps |xc| in (7.5 * 2^-9, 2^-6) at 7 * 2^-9 where the hardware rounds up
-// to 2^-6; clamping those to 7 * 2^-9 first makes the two agree.  NaN stays
-// NaN (the conversion then gives a NaN byte, of either sign).
-__device__ __forceinline__ float fp8_prerounded(float x, float inv) {
-    const float xs = x * inv;
-    const float xc = __builtin_amdgcn_fmed3f(xs, -448.0f, 448.0f);   // xs not NaN
+// to 2^-6; clamping those to 7 * 2^-9 first makes the two agree.  xs is not
+// NaN (the hardware's NaN byte is not the codec's).
+__device__ __forceinline__ float fp8_prerounded(float xs) {
+    const float xc = __builtin_amdgcn_fmed3f(xs, -448.0f, 448.0f);
     const float sub = __builtin_amdgcn_fmed3f(xc, -7.0f * 0x1p-9f, 7.0f * 0x1p-9f);
-    const float v = fabsf(xc) < 0x1p-6f ? sub : xc;
-    return __builtin_isnan(xs) ? xs : v;
+    return fabsf(xc) < 0x1p-6f ? sub : xc;
 }
 
-// Four E4M3 bytes of a lane's four values, low byte first.
+// The bytes fp8_quant(x[e], inv) of a lane's four values, low byte first.
 __device__ __forceinline__ uint32_t fp8_pack4(v4f x, float inv) {
-    int w = __builtin_amdgcn_cvt_pk_fp8_f32(fp8_prerounded(x[0], inv), fp8_prerounded(x[1], inv), 0, false);
-    w = __builtin_amdgcn_cvt_pk_fp8_f32(fp8_prerounded(x[2], inv), fp8_prerounded(x[3], inv), w, true);
+    float xs[4];
+    bool nan = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        xs[e] = x[e] * inv;
+        nan |= __builtin_isnan(xs[e]);
+    }
+    int w = __builtin_amdgcn_cvt_pk_fp8_f32(fp8_prerounded(xs[0]), fp8_prerounded(xs[1]), 0, false);
+    w = __builtin_amdgcn_cvt_pk_fp8_f32(fp8_prerounded(xs[2]), fp8_prerounded(xs[3]), w, true);
+    if (nan) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (__builtin_isnan(xs[e])) w = (w & ~(0xFF << (8 * e))) | (0x7F << (8 * e));
+    }
     return static_cast<uint32_t>(w);
 }
 

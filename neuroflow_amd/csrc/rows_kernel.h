@@ -433,6 +433,7 @@ __global__ __launch_bounds__(256, rows_min_waves(KB, FP8)) void k_rows(RowsArgs 
             if constexpr (OUT == OUT_EPI) srow = row_ok ? a.scale_in[row] : 1.0f;
         } else {
             float inv;
+            const bool fixed_fast = a.scale_A >= 0x1p-120f && a.scale_A <= 0x1p120f;
             if constexpr (IN == IN_F32_TOKEN) {
                 float mx = 0.0f;
 #pragma unroll
@@ -456,7 +457,7 @@ __global__ __launch_bounds__(256, rows_min_waves(KB, FP8)) void k_rows(RowsArgs 
                 }
             } else {
                 srow = a.scale_A;
-                inv = FP8 ? ((srow == 0.0f) ? 1.0f : 1.0f / srow) : 0.0f;
+                inv = 1.0f / srow;
             }
             if constexpr (FP8) {
 #pragma unroll
@@ -495,10 +496,7 @@ __global__ __launch_bounds__(256, rows_min_waves(KB, FP8)) void k_rows(RowsArgs 
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         const v4f v = cur.x[kb][j];
-                        xc[kb][j] = pack4(quant_i8_exact(v[0], srow, a.zp_A),
-                                          quant_i8_exact(v[1], srow, a.zp_A),
-                                          quant_i8_exact(v[2], srow, a.zp_A),
-                                          quant_i8_exact(v[3], srow, a.zp_A));
+                        xc[kb][j] = quant_i8_fixed4(v, srow, inv, a.zp_A, fixed_fast);
                         // Padding beyond K must stay 0 even when zp_A != 0.
                         const int k = kb * 64 + j * 16 + g * 4;
                         if (!(row_ok && k < K)) xc[kb][j] = 0u;

@@ -174,19 +174,7 @@ __device__ __forceinline__ void token_quantise_row(const RowsArgs& a, const v4f 
                 v = pack4(quant_i8_token(x[j][0], s, inv), quant_i8_token(x[j][1], s, inv),
                           quant_i8_token(x[j][2], s, inv), quant_i8_token(x[j][3], s, inv));
             } else {
-                int32_t c[4];
-                bool any_bad = !fast;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    bool bad;
-                    c[e] = quant_i8_fixed_near(x[j][e], inv, a.zp_A, bad);
-                    any_bad |= bad;
-                }
-                v = pack4(c[0], c[1], c[2], c[3]);
-                if (any_bad) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v = patch_fixed_code(v, x[j][e], e, s, a.zp_A);
-                }
+                v = quant_i8_fixed4(x[j], s, inv, a.zp_A, fast);
                 if constexpr (RAG) v = token_mask_codes(v, a.K - (4 * r + 64 * j));
             }
             v = live ? v : 0u;
