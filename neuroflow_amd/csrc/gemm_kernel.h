@@ -114,8 +114,8 @@ __device__ __forceinline__ bool gemm_epi_tables(const RowsArgs& a, int n0, ColSu
 // reads it back row-contiguously, so each store instruction writes
 // 64 / (4 TN) rows of 64 TN contiguous bytes.  srow[i] / sa[i]: the row
 // scale and row code sum of lane row i.
-template <int TM, int TN, int OUT, int ACT>
-__device__ __forceinline__ void gemm_store(const RowsArgs& a, const v4i (&acc)[TM][TN], int64_t m0,
+template <int TM, int TN, int OUT, int ACT, typename Acc>
+__device__ __forceinline__ void gemm_store(const RowsArgs& a, const Acc (&acc)[TM][TN], int64_t m0,
                                            int n0, int wm, int wn, uint32_t* strip,
                                            const float (&srow)[TM], const int32_t (&sa)[TM],
                                            bool trivial, const IntEpi* lds_e, const float* lds_scw,
@@ -149,7 +149,7 @@ __device__ __forceinline__ void gemm_store(const RowsArgs& a, const v4i (&acc)[T
                 } else {
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
-                        const float t = int_epi_value(lds_e[lcol + v], acc[i][j][v], sa[i]);
+                        const float t = int_epi_value(lds_e[lcol + v], static_cast<int32_t>(acc[i][j][v]), sa[i]);
                         y[v] = activate<ACT>(dequant_bias(swv[v], srow[i], t, bv[v]));
                     }
                 }
@@ -430,8 +430,14 @@ __device__ __forceinline__ void gemm_stage_sync() {
 // MF selects the MFMA: 16 (v_mfma_i32_16x16x64_i8, TM x TN tiles of 16 x 16
 // per wave) or 32 (v_mfma_i32_32x32x32_i8, (TM / 2) x (TN / 2) tiles of
 // 32 x 32: half the operand reads per product and a higher issue rate).
-template <int TM, int TN, int OUT, int ACT, int MF = 16>
+//
+// FP8: E4M3 codes on both sides.  They stay bytes in HBM and LDS (half the
+// traffic of bf16 operands) and become bf16 in registers, a fragment of 16
+// bytes feeding two v_mfma_f32_16x16x32_bf16; per K step a wave converts
+// 8 (TM + TN) registers beside 2 TM TN MFMAs.
+template <int TM, int TN, int OUT, int ACT, int MF = 16, bool FP8 = false>
 __global__ __launch_bounds__(256, 2) void k_gemm_pipe(RowsArgs a, int xcd_groups) {
+    static_assert(!FP8 || MF == 16, "FP8 uses the 16 x 16 tiles");
     static_assert(MF == 16 || (MF == 32 && TM % 2 == 0 && TN % 2 == 0), "32 x 32 tiles need even TM, TN");
     using S = GemmShape<TM, TN>;
     constexpr int BM = S::BM, BN = S::BN;
@@ -485,7 +491,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_pipe(RowsArgs a, int xcd_groups
     };
 
     constexpr int AI = MF == 32 ? TM / 2 : TM, AJ = MF == 32 ? TN / 2 : TN;
-    using Acc = std::conditional_t<MF == 32, v16i, v4i>;
+    using Acc = std::conditional_t<FP8, v4f, std::conditional_t<MF == 32, v16i, v4i>>;
     Acc acc[AI][AJ];
 #pragma unroll
     for (int i = 0; i < AI; ++i)
@@ -525,6 +531,23 @@ __global__ __launch_bounds__(256, 2) void k_gemm_pipe(RowsArgs a, int xcd_groups
 #pragma unroll
         for (int j = 0; j < TN; ++j)
             wf[j] = *reinterpret_cast<const v4i*>(cur + BM * GEMM_LDS_ROW + gemm_lds_off(16 * TN * wn + 16 * j + r, g));
+        if constexpr (FP8) {
+            v8bf xb[TM][2];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                xb[i][0] = fp8x8_to_bf16(xf[i][0], xf[i][1]);
+                xb[i][1] = fp8x8_to_bf16(xf[i][2], xf[i][3]);
+            }
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const v8bf w0 = fp8x8_to_bf16(wf[j][0], wf[j][1]), w1 = fp8x8_to_bf16(wf[j][2], wf[j][3]);
+#pragma unroll
+                for (int i = 0; i < TM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0, xb[i][0], acc[i][j], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < TM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1, xb[i][1], acc[i][j], 0, 0, 0);
+            }
+            return;
+        } else {
         __builtin_amdgcn_sched_group_barrier(0x0100, TM + TN, 0);  // DS reads
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -532,6 +555,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_pipe(RowsArgs a, int xcd_groups
             for (int j = 0; j < TN; ++j)
                 acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[j], xf[i], acc[i][j], 0, 0, 0);
         __builtin_amdgcn_sched_group_barrier(0x0008, TM * TN, 0);  // MFMA
+        }
         }
     };
 

@@ -39,13 +39,12 @@ static void launch_rows_kb(const RowsArgs& a, hipStream_t st) {
 template <bool FP8, int IN, int OUT, int ACT>
 static void launch_rows_act(const RowsArgs& a, hipStream_t st) {
     const int kb = (a.K + 63) / 64;
-    if (kb <= 1) launch_rows_kb<1, FP8, IN, OUT, ACT>(a, st);
-    else if (IN == IN_CODES || rows_hoist_fits(2, FP8)) {
-        if (kb <= 2) launch_rows_kb<2, FP8, IN, OUT, ACT>(a, st);
-    }
-    if constexpr (IN == IN_CODES) {
-        if (kb <= 2) return;
-        if (kb <= 4) launch_rows_kb<4, FP8, IN, OUT, ACT>(a, st);
+    if constexpr (IN != IN_CODES) {
+        launch_rows_kb<1, FP8, IN, OUT, ACT>(a, st);   // K <= 64 (rows_ok)
+    } else {
+        if (kb <= 1) launch_rows_kb<1, FP8, IN, OUT, ACT>(a, st);
+        else if (kb <= 2) launch_rows_kb<2, FP8, IN, OUT, ACT>(a, st);
+        else if (kb <= 4) launch_rows_kb<4, FP8, IN, OUT, ACT>(a, st);
         else if (kb <= 8) launch_rows_kb<8, FP8, IN, OUT, ACT>(a, st);
         else launch_rows_kb<16, FP8, IN, OUT, ACT>(a, st);
     }

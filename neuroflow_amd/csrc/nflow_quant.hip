@@ -593,9 +593,9 @@ static int formula_row(int K) { return K <= 4096 ? F_ROW_VNNI : F_ROW_SCALAR; }
 // rather than the row-tile kernel or the generic one.  The row-tile kernel
 // stays where it can run (weights in registers: 300000 x 64 -> 40 26.9 us
 // either way).
-static bool use_token_gemm(const RowsArgs& a, bool fp8) {
+static bool use_token_gemm(const RowsArgs& a) {
     if (!token_gemm_ok(a) || path_flag(kernel_path().no_token_gemm)) return false;
-    return !rows_ok(a, IN_F32_TOKEN, fp8);
+    return !rows_ok(a, IN_F32_TOKEN);
 }
 
 // Per-token INT8 shapes the tiled GEMM could also take (after a quantise
@@ -617,6 +617,15 @@ static bool split_faster(const RowsArgs& a) {
     if (a.M < 16384) return true;
     if (a.N <= 256) return false;
     return a.M < 32768 || (a.K == 512 && a.N > 512 && a.N % 32 == 0);
+}
+
+// The same choice for FP8 (K >= 512).  Measured on MI355X (us, one-pass /
+// split): 1000 x 1024 -> 1024 17 / 11, 4096 x 1024 -> 1024 40 / 21; at K = 512
+// 1000 -> 1024 10.2 / 9.5, 16384 -> 256 14.3 / 20.9, 16384 -> 1024 30 / 34.7, but
+// 20000 -> 2048 79 / 64.
+static bool fp8_split_faster(const RowsArgs& a) {
+    if (kernel_path().token_rows.load(std::memory_order_relaxed)) return false;   // forced tiles: one-pass
+    return a.K > 512 || (a.N > 1024 && !token_small_tiles(a));
 }
 
 // Fixed-scale int8 path shared by LinearForward / rows / batched.
@@ -641,7 +650,7 @@ static int int8_fixed_path(const nflow_int8_linear_params* p, int64_t rows, cons
         launch_rows64_fixed(a, st);
         return check_launch(what);
     }
-    if (use_token_gemm(a, false)) {
+    if (use_token_gemm(a)) {
         launch_token_i8_fixed(a, st);
         return check_launch(what);
     }
@@ -916,7 +925,7 @@ static int int8_per_token(const nflow_int8_linear_params* p, int64_t M, const fl
     RowsArgs g = a;
     g.Aq = nullptr;  // the codes go to the workspace, which is 256-byte aligned
     const bool wide = use_gemm(g);
-    if (use_token_gemm(a, false) && !(wide && split_faster(a)) && !(fixed && noalloc_refuses(a, wide, fixed->cap))) {
+    if (use_token_gemm(a) && !(wide && split_faster(a)) && !(fixed && noalloc_refuses(a, wide, fixed->cap))) {
         launch_token_i8(a, act_x2, st);
         return finish();
     }
@@ -1160,11 +1169,16 @@ static int fp8_per_token(const nflow_fp8_linear_params* p, int64_t M, const floa
         if (post) hipLaunchKernelGGL(k_fno_post, dim3(grid_for(M, 1, 16)), dim3(256), 0, st, C, R, a, activation);
         return check_launch("fp8_linear_forward_per_token");
     };
-    if (use_token_gemm(a, true)) {
+    // K a multiple of 64, at least 512: quantise, then the tiled GEMM, where
+    // that is the faster form.
+    RowsArgs g = a;
+    g.Aq = nullptr;  // the codes go to the workspace, which is 256-byte aligned
+    const bool wide = a.K >= 512 && use_gemm(g);
+    if (use_token_gemm(a) && !(wide && fp8_split_faster(a))) {
         launch_token_fp8(a, act_x2, st);
         return finish();
     }
-    if (rows_ok(a, IN_F32_TOKEN, true)) {
+    if (rows_ok(a, IN_F32_TOKEN)) {
         launch_rows<true, IN_F32_TOKEN, OUT_EPI>(a, act_x2, st);
         return finish();
     }
@@ -1177,7 +1191,8 @@ static int fp8_per_token(const nflow_fp8_linear_params* p, int64_t M, const floa
     if (scale_A_out) (void)hipMemcpyAsync(scale_A_out, sc, sizeof(float) * M, hipMemcpyDeviceToDevice, st);
     a.Aq = q;
     a.scale_in = sc;
-    if (rows_ok(a, IN_CODES)) launch_rows<true, IN_CODES, OUT_EPI>(a, act_x2, st);
+    if (wide) launch_gemm_fp8<OUT_EPI>(a, act_x2, st);
+    else if (rows_ok(a, IN_CODES)) launch_rows<true, IN_CODES, OUT_EPI>(a, act_x2, st);
     else launch_generic<true, OUT_EPI>(a, act_x2, st);
     return finish();
 }
@@ -1220,7 +1235,8 @@ int nflow_fp8_gemm_f32(const uint8_t* A_q, const uint8_t* W_q, int64_t M, int N,
     a.W = W_q;
     a.kb_dot = (K + 63) / 64;
     a.C = C;
-    if (rows_ok(a, IN_CODES)) launch_rows<true, IN_CODES, OUT_RAW>(a, ACT_NONE, as_stream(stream));
+    if (use_gemm(a)) launch_gemm_fp8<OUT_RAW>(a, ACT_NONE, as_stream(stream));
+    else if (rows_ok(a, IN_CODES)) launch_rows<true, IN_CODES, OUT_RAW>(a, ACT_NONE, as_stream(stream));
     else launch_generic<true, OUT_RAW>(a, ACT_NONE, as_stream(stream));
     return check_launch("fp8_gemm_f32");
 }
@@ -1244,7 +1260,8 @@ int nflow_fp8_linear_forward_quantised(const nflow_fp8_linear_params* p, int64_t
     a.bias = p->bias;
     a.kb_dot = (a.K + 63) / 64;
     a.C = C;
-    if (rows_ok(a, IN_CODES)) launch_rows<true, IN_CODES, OUT_EPI>(a, activation, as_stream(stream));
+    if (use_gemm(a)) launch_gemm_fp8<OUT_EPI>(a, activation, as_stream(stream));
+    else if (rows_ok(a, IN_CODES)) launch_rows<true, IN_CODES, OUT_EPI>(a, activation, as_stream(stream));
     else launch_generic<true, OUT_EPI>(a, activation, as_stream(stream));
     return check_launch("fp8_linear_forward_quantised");
 }
