@@ -363,8 +363,13 @@ __device__ __forceinline__ IntEpi int_epi_consts(int formula, int32_t K, int32_t
 __device__ __forceinline__ float int_epi_value(const IntEpi& e, int32_t D, int32_t SA) {
     const uint32_t t32 = static_cast<uint32_t>(D) + static_cast<uint32_t>(e.c0) +
                          static_cast<uint32_t>(e.c1) * static_cast<uint32_t>(SA);
-    if (e.c2 == 0) return static_cast<float>(static_cast<int32_t>(t32));
-    return static_cast<float>(static_cast<int64_t>(static_cast<int32_t>(t32)) + e.c2);
+    // The 64-bit sum as a 32-bit one wherever that holds it (the conversion
+    // to float then rounds the same integer): the 64-bit conversion costs
+    // several times the rest of the epilogue.
+    const int32_t t = static_cast<int32_t>(t32), c2 = static_cast<int32_t>(e.c2);
+    int32_t u;
+    if (c2 == e.c2 && !__builtin_add_overflow(t, c2, &u)) return static_cast<float>(u);
+    return static_cast<float>(static_cast<int64_t>(t) + e.c2);
 }
 
 // The FNO layer's INT8 fake-quant of x2 (fno.cpp:626-646 per-position,

@@ -26,18 +26,19 @@ static void launch_gemm_t(const RowsArgs& a, hipStream_t st) {
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(256), lds, st, a, groups);
 }
 
-// Tile shape: 128 x 256 for large M and N (two blocks per CU); 64 x 128 for
-// M <= 4096 with N >= 512 (twice the blocks of 128 x 128: at C5's branch,
-// M = 4096, K = N = 1024, 12.6 us against 13.7 us, and 14.2 us at 64 x 64);
-// else 128 x 128.  Measured on MI355X: 256 x 256 (one wave per SIMD) never
-// beats 128 x 256, 64 x 128 loses at the trunk (173 us against 139 us).
+// Tile shape: 128 x 256 for large M and N (two blocks per CU), else 128 x 128
+// where that gives every CU a block, else 64 x 64 (four times the blocks, and
+// a lone block's K steps take half the time).  Measured on MI355X: 256 x 256
+// (one wave per SIMD) never beats 128 x 256; static 4096 x 1024 -> 256 with its
+// quantise 22.5 us at 128 x 128, 13.9 at 64 x 64.
 static int gemm_shape(const RowsArgs& a) {
     // A gemm_tile override of 88|48|44|24|22 forces a shape (for tile sweeps;
     // 22 and 24 only on the LDS-DMA kernel).
     const int t = kernel_path().gemm_tile.load(std::memory_order_relaxed);
     if (t == 88 || t == 48 || t == 44 || t == 22 || t == 24) return t;
     if (a.M >= 16384 && a.N >= 1024) return 48;
-    return (a.M <= 4096 && a.N >= 512) ? 24 : 44;
+    const int64_t blocks = ((a.M + 127) / 128) * ((static_cast<int64_t>(a.N) + 127) / 128);
+    return a.N <= 64 || blocks < num_cus() ? 22 : 44;
 }
 
 template <int TM, int TN, int OUT, int ACT>
@@ -54,14 +55,18 @@ static void launch_pipe_t(const RowsArgs& a, hipStream_t st) {
                            a, groups);
 }
 
+// Whether the formula's integer terms take the weight-row byte sums.
+bool gemm_needs_colsum(const RowsArgs& a) {
+    return (a.formula == F_ROW_VNNI && (a.sumW || a.zp_A != 0)) || (a.formula == F_ROW_SCALAR && a.zp_A != 0);
+}
+
 // The LDS-DMA kernel takes every case whose epilogue needs no byte sums of
-// its own: zp_A = 0, row sums given when zero points may be nonzero, and
-// weight-row sums given when the row-VNNI formula has a caller's sum_W.
+// its own: row sums given when zero points may be nonzero, and weight-row
+// sums given when the formula takes them.
 bool gemm_pipe_ok(const RowsArgs& a, int out) {
-    if (a.zp_A != 0 || path_flag(kernel_path().gemm_reg)) return false;
+    if (path_flag(kernel_path().gemm_reg)) return false;
     if (out == OUT_RAW) return true;
-    const bool need_colsum = a.formula == F_ROW_VNNI && a.sumW;
-    return (!a.zpW || a.sum_in) && (!need_colsum || a.colsum_in);
+    return (!a.zpW || a.sum_in) && (!gemm_needs_colsum(a) || a.colsum_in);
 }
 
 // The persistent GEMM (wide_kernel.h): the fused epilogue with zp_A = 0 and

@@ -53,6 +53,7 @@ struct KernelPath {
     std::atomic<int> no_rows64{0};
     std::atomic<int> no_token_gemm{0};
     std::atomic<int> token_rows{0};  // 0: the launcher's choice, else 16 or 64 rows per tile
+    std::atomic<int> skinny{0};      // 0: the launcher's choice, 1: wherever it can run, 2: never
     std::atomic<int> gemm_reg{0};
     std::atomic<int> gemm_tile{0};   // 0: the launcher's choice
     std::atomic<int> gemm_mfma{0};   // 0: the launcher's choice, else 16 or 32
@@ -111,10 +112,18 @@ void launch_token_i8(const RowsArgs& a, int act, hipStream_t st);
 void launch_token_i8_fixed(const RowsArgs& a, hipStream_t st);
 void launch_token_fp8(const RowsArgs& a, int act, hipStream_t st);
 
+// The few-row layer (skinny.hip): K split over a block's waves.
+bool skinny_ok(const RowsArgs& a);
+void launch_skinny_i8(const RowsArgs& a, int act, hipStream_t st);
+void launch_skinny_i8_fixed(const RowsArgs& a, hipStream_t st);
+void launch_skinny_fp8(const RowsArgs& a, int act, hipStream_t st);
+
 // The tiled MFMA GEMM on INT8 codes for K a multiple of 64, K >= 128 (gemm.hip).
 bool gemm_ok(const RowsArgs& a);
 // Whether launch_gemm takes the LDS-DMA kernel for `a` (out: OUT_EPI / OUT_RAW).
 bool gemm_pipe_ok(const RowsArgs& a, int out);
+// Whether the formula's integer terms take the weight-row byte sums.
+bool gemm_needs_colsum(const RowsArgs& a);
 template <int OUT>
 void launch_gemm(const RowsArgs& a, int act, hipStream_t st);
 // The same on E4M3 codes (gemm_fp8.hip): the LDS-DMA kernel whenever gemm_ok.

@@ -116,6 +116,39 @@ __device__ __forceinline__ void code_sums_share(const CodeSums& cs) {
         code_sums_group(cs, wg);
 }
 
+// Codes of (M, K) rows with one scale (K a multiple of 4, 16-byte aligned
+// rows) and their row sums, for the tiled GEMM: a wave per row, four float4
+// per lane in flight.  Bound by HBM.
+__global__ __launch_bounds__(256) void k_quantise_fixed_rows(const float* __restrict__ A, int64_t M, int K,
+                                                             uint8_t* __restrict__ Aq, int32_t* __restrict__ sum_a,
+                                                             float s, int32_t zp, CodeSums cs) {
+    code_sums_share(cs);
+    const int lane = threadIdx.x & 63, kq = K / 4;
+    const float inv = 1.0f / s;
+    const bool fast = s >= 0x1p-120f && s <= 0x1p120f;   // the reciprocal path's range
+    const int64_t nw = static_cast<int64_t>(gridDim.x) * 4;
+    for (int64_t m = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6); m < M; m += nw) {
+        const v4f* x4 = reinterpret_cast<const v4f*>(A + m * K);
+        uint32_t* q4 = reinterpret_cast<uint32_t*>(Aq + m * K);
+        int32_t sa = 0;
+        for (int j = lane; j < kq; j += 256) {
+            v4f x[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) x[u] = __builtin_nontemporal_load(x4 + (j + 64 * u < kq ? j + 64 * u : j));
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if (j + 64 * u >= kq) continue;
+                const uint32_t v = quant_i8_fixed4(x[u], s, inv, zp, fast);
+                q4[j + 64 * u] = v;
+                sa = sum_bytes_i8(v, sa);
+            }
+        }
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) sa += __shfl_xor(sa, o);
+        if (lane == 0) sum_a[m] = sa;
+    }
+}
+
 template <bool FP8>
 __global__ __launch_bounds__(256) void k_quantise_token(const float* __restrict__ A, int64_t M,
                                                         int K, uint8_t* __restrict__ Aq,
@@ -589,6 +622,10 @@ static int kb_dot_for(int formula, int K) {
 
 static int formula_row(int K) { return K <= 4096 ? F_ROW_VNNI : F_ROW_SCALAR; }
 
+// The tiled GEMM serves INT8 code input with K a multiple of 64, K >= 128
+// (NFLOW_NO_GEMM=1 selects the row-tile kernel instead, for A/B timing).
+static bool use_gemm(const RowsArgs& a) { return gemm_ok(a) && !path_flag(kernel_path().no_gemm); }
+
 // Whether a layer on fp32 input takes the one-pass kernel (token_gemm_kernel.h)
 // rather than the row-tile kernel or the generic one.  The row-tile kernel
 // stays where it can run (weights in registers: 300000 x 64 -> 40 26.9 us
@@ -596,6 +633,25 @@ static int formula_row(int K) { return K <= 4096 ? F_ROW_VNNI : F_ROW_SCALAR; }
 static bool use_token_gemm(const RowsArgs& a) {
     if (!token_gemm_ok(a) || path_flag(kernel_path().no_token_gemm)) return false;
     return !rows_ok(a, IN_F32_TOKEN);
+}
+
+// Whether a layer on fp32 input takes the few-row kernel (skinny_kernel.h):
+// while its 16 x 16 output blocks, which each quantise their rows for
+// themselves, are few.  Measured on MI355X (us, few-row / the kernel that
+// runs otherwise): static 1 x 1024 -> 1024 5.2 / 12.6, INT8 64 x 1024 -> 1024
+// (256 blocks) 7.1 / 11.1, 128 x (512 blocks) 12.2 / 11.3; K <= 256 (4 waves
+// per block) 300 x 200 -> 512 (608 blocks) 5.1 / 7.1, 2000 x 256 -> 64 (500)
+// 4.9 / 5.5, 1000 x 256 -> 256 (1008) 6.4 / 5.5; K <= 128, where the one-pass
+// kernel's chain is short, 300 x 64 -> 128 (152) 4.0 / 3.7; K = 4096, 1 -> 2048
+// (128) 13 / 19, 128 rows (1024) 67 / 21.
+static bool use_skinny(const RowsArgs& a) {
+    const int f = kernel_path().skinny.load(std::memory_order_relaxed);
+    if (f == 2 || !skinny_ok(a)) return false;
+    if (f == 1) return true;
+    const int64_t blocks = ((a.M + 15) / 16) * ((static_cast<int64_t>(a.N) + 15) / 16);
+    const int64_t cus = num_cus();
+    if (a.K <= 128 || a.K > 2048) return blocks <= cus / 2;
+    return blocks <= (a.K <= 256 ? 2 * cus : cus);
 }
 
 // Per-token INT8 shapes the tiled GEMM could also take (after a quantise
@@ -628,6 +684,15 @@ static bool fp8_split_faster(const RowsArgs& a) {
     return a.K > 512 || (a.N > 1024 && !token_small_tiles(a));
 }
 
+// The same choice for fixed-scale INT8.  Measured on MI355X (us, one-pass /
+// split): K = 320 16384 -> 256 18.2 / 22.6, -> 1024 41.1 / 40.5; K = 512 4096 ->
+// 1024 21.6 / 19.4, 8192 -> 2048 38.4 / 41.4, 16384 -> 256 21.3 / 27.1; K = 1024
+// 300 -> 256 13.6 / 11.6, 4096 -> 1024 44 / 23, 16384 -> 1024 151 / 58.
+static bool fixed_split_faster(const RowsArgs& a) {
+    if (kernel_path().token_rows.load(std::memory_order_relaxed)) return false;   // forced tiles: one-pass
+    return a.K > 512;
+}
+
 // Fixed-scale int8 path shared by LinearForward / rows / batched.
 static int int8_fixed_path(const nflow_int8_linear_params* p, int64_t rows, const float* A, float* C,
                            int formula, hipStream_t st, const char* what) {
@@ -646,12 +711,37 @@ static int int8_fixed_path(const nflow_int8_linear_params* p, int64_t rows, cons
     a.formula = formula;
     a.kb_dot = kb_dot_for(formula, a.K);
     a.C = C;
+    if (use_skinny(a)) {
+        launch_skinny_i8_fixed(a, st);
+        return check_launch(what);
+    }
     if (rows64_ok(a) && !path_flag(kernel_path().no_rows64)) {
         launch_rows64_fixed(a, st);
         return check_launch(what);
     }
-    if (use_token_gemm(a)) {
+    RowsArgs g = a;
+    g.Aq = nullptr;  // the codes go to the workspace, which is 256-byte aligned
+    const bool wide = aligned(A, 16) && use_gemm(g);
+    if (use_token_gemm(a) && !(wide && fixed_split_faster(a))) {
         launch_token_i8_fixed(a, st);
+        return check_launch(what);
+    }
+    if (wide) {
+        // Quantise (with the row sums, and the weight-row sums where the
+        // formula takes them), then the tiled GEMM.
+        const bool want_colsum = gemm_needs_colsum(a);
+        const size_t codes16 = ((static_cast<size_t>(rows) * a.K + 15) / 16) * 16;
+        Scratch ws(codes16 + (static_cast<size_t>(rows) + (want_colsum ? a.N : 0)) * sizeof(int32_t), st);
+        if (ws.err != hipSuccess) return set_error(NFLOW_INTERNAL, std::string(what) + ": workspace allocation failed");
+        uint8_t* q = static_cast<uint8_t*>(ws.p);
+        int32_t* sums = reinterpret_cast<int32_t*>(q + codes16);
+        int32_t* colsum = want_colsum ? sums + rows : nullptr;
+        hipLaunchKernelGGL(k_quantise_fixed_rows, dim3(grid_for(rows, 4, 16)), dim3(256), 0, st, A, rows, a.K, q, sums,
+                           p->scale_A, p->zp_A, CodeSums{a.W, a.N, a.K, colsum});
+        a.Aq = q;
+        a.sum_in = sums;
+        a.colsum_in = colsum;
+        launch_gemm<OUT_EPI>(a, ACT_NONE, st);
         return check_launch(what);
     }
     if (rows_ok(a, IN_F32_FIXED)) {
@@ -668,10 +758,6 @@ static int int8_fixed_path(const nflow_int8_linear_params* p, int64_t rows, cons
     launch_generic<false, OUT_EPI>(a, ACT_NONE, st);
     return check_launch(what);
 }
-
-// The tiled GEMM serves INT8 code input with K a multiple of 64, K >= 128
-// (NFLOW_NO_GEMM=1 selects the row-tile kernel instead, for A/B timing).
-static bool use_gemm(const RowsArgs& a) { return gemm_ok(a) && !path_flag(kernel_path().no_gemm); }
 
 static int check_params(const nflow_int8_linear_params* p, const char* what) {
     if (!p || !p->W_int8 || !p->scale_W || !p->zp_W)
@@ -700,6 +786,7 @@ int nflow_debug_set_kernel_path(const char* name, int value, int* previous) {
                         : n == "no_rows64" ? &k.no_rows64
                         : n == "no_token_gemm" ? &k.no_token_gemm
                         : n == "token_rows" ? &k.token_rows
+                        : n == "skinny" ? &k.skinny
                         : n == "gemm_reg" ? &k.gemm_reg
                         : n == "gemm_tile" ? &k.gemm_tile
                         : n == "gemm_mfma" ? &k.gemm_mfma
@@ -925,7 +1012,12 @@ static int int8_per_token(const nflow_int8_linear_params* p, int64_t M, const fl
     RowsArgs g = a;
     g.Aq = nullptr;  // the codes go to the workspace, which is 256-byte aligned
     const bool wide = use_gemm(g);
-    if (use_token_gemm(a) && !(wide && split_faster(a)) && !(fixed && noalloc_refuses(a, wide, fixed->cap))) {
+    const bool refused = fixed && noalloc_refuses(a, wide, fixed->cap);
+    if (!refused && use_skinny(a)) {
+        launch_skinny_i8(a, act_x2, st);
+        return finish();
+    }
+    if (!refused && use_token_gemm(a) && !(wide && split_faster(a))) {
         launch_token_i8(a, act_x2, st);
         return finish();
     }
@@ -1169,6 +1261,10 @@ static int fp8_per_token(const nflow_fp8_linear_params* p, int64_t M, const floa
         if (post) hipLaunchKernelGGL(k_fno_post, dim3(grid_for(M, 1, 16)), dim3(256), 0, st, C, R, a, activation);
         return check_launch("fp8_linear_forward_per_token");
     };
+    if (use_skinny(a)) {
+        launch_skinny_fp8(a, act_x2, st);
+        return finish();
+    }
     // K a multiple of 64, at least 512: quantise, then the tiled GEMM, where
     // that is the faster form.
     RowsArgs g = a;
