@@ -120,8 +120,9 @@ __device__ __forceinline__ void code_sums_share(const CodeSums& cs) {
 // rows) and their row sums, for the tiled GEMM: a wave per row, four float4
 // per lane in flight.  Bound by HBM.
 __global__ __launch_bounds__(256) void k_quantise_fixed_rows(const float* __restrict__ A, int64_t M, int K,
-                                                             uint8_t* __restrict__ Aq, int32_t* __restrict__ sum_a,
-                                                             float s, int32_t zp, CodeSums cs) {
+                                                             uint8_t* __restrict__ Aq, float* __restrict__ scale,
+                                                             int32_t* __restrict__ sum_a, float s, int32_t zp,
+                                                             CodeSums cs) {
     code_sums_share(cs);
     const int lane = threadIdx.x & 63, kq = K / 4;
     const float inv = 1.0f / s;
@@ -145,7 +146,10 @@ __global__ __launch_bounds__(256) void k_quantise_fixed_rows(const float* __rest
         }
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) sa += __shfl_xor(sa, o);
-        if (lane == 0) sum_a[m] = sa;
+        if (lane == 0) {
+            sum_a[m] = sa;
+            scale[m] = s;      // the persistent GEMM reads its rows' scales
+        }
     }
 }
 
@@ -685,12 +689,14 @@ static bool fp8_split_faster(const RowsArgs& a) {
 }
 
 // The same choice for fixed-scale INT8.  Measured on MI355X (us, one-pass /
-// split): K = 320 16384 -> 256 18.2 / 22.6, -> 1024 41.1 / 40.5; K = 512 4096 ->
-// 1024 21.6 / 19.4, 8192 -> 2048 38.4 / 41.4, 16384 -> 256 21.3 / 27.1; K = 1024
-// 300 -> 256 13.6 / 11.6, 4096 -> 1024 44 / 23, 16384 -> 1024 151 / 58.
+// split): K = 320 16384 -> 256 18.2 / 22.6, -> 1024 41.1 / 40.5; K = 512, where
+// the split runs the persistent GEMM, 1000 -> 512 9.9 / 10.8, 4096 -> 256 11.8 /
+// 12.1, -> 512 16.2 / 12.5, 8192 -> 2048 41.6 / 30.2, 65536 -> 256 55.4 / 58.6;
+// K = 1024 300 -> 256 13.6 / 11.6, 4096 -> 1024 44 / 17.4, 16384 -> 1024 150 / 45.
 static bool fixed_split_faster(const RowsArgs& a) {
     if (kernel_path().token_rows.load(std::memory_order_relaxed)) return false;   // forced tiles: one-pass
-    return a.K > 512;
+    const int64_t pairs = ((a.M + 15) / 16) * ((static_cast<int64_t>(a.N) + 127) / 128);
+    return a.K > 512 || (a.K == 512 && a.N >= 512 && pairs > 2 * static_cast<int64_t>(num_cus()));
 }
 
 // Fixed-scale int8 path shared by LinearForward / rows / batched.
@@ -731,14 +737,16 @@ static int int8_fixed_path(const nflow_int8_linear_params* p, int64_t rows, cons
         // formula takes them), then the tiled GEMM.
         const bool want_colsum = gemm_needs_colsum(a);
         const size_t codes16 = ((static_cast<size_t>(rows) * a.K + 15) / 16) * 16;
-        Scratch ws(codes16 + (static_cast<size_t>(rows) + (want_colsum ? a.N : 0)) * sizeof(int32_t), st);
+        Scratch ws(codes16 + (2 * static_cast<size_t>(rows) + (want_colsum ? a.N : 0)) * sizeof(int32_t), st);
         if (ws.err != hipSuccess) return set_error(NFLOW_INTERNAL, std::string(what) + ": workspace allocation failed");
         uint8_t* q = static_cast<uint8_t*>(ws.p);
-        int32_t* sums = reinterpret_cast<int32_t*>(q + codes16);
+        float* sc = reinterpret_cast<float*>(q + codes16);
+        int32_t* sums = reinterpret_cast<int32_t*>(sc + rows);
         int32_t* colsum = want_colsum ? sums + rows : nullptr;
-        hipLaunchKernelGGL(k_quantise_fixed_rows, dim3(grid_for(rows, 4, 16)), dim3(256), 0, st, A, rows, a.K, q, sums,
-                           p->scale_A, p->zp_A, CodeSums{a.W, a.N, a.K, colsum});
+        hipLaunchKernelGGL(k_quantise_fixed_rows, dim3(grid_for(rows, 4, 16)), dim3(256), 0, st, A, rows, a.K, q, sc,
+                           sums, p->scale_A, p->zp_A, CodeSums{a.W, a.N, a.K, colsum});
         a.Aq = q;
+        a.scale_in = sc;
         a.sum_in = sums;
         a.colsum_in = colsum;
         launch_gemm<OUT_EPI>(a, ACT_NONE, st);

@@ -193,7 +193,11 @@ constexpr int wide_wait(int k, int nk, int nl, int ntab, int stores, int lead) {
 // s_waitcnt with vmcnt = n (gfx9 split field), expcnt off, lgkmcnt = 0.
 constexpr int wide_waitcnt_imm(int n) { return 0x070 | (n & 15) | ((n >> 4) << 14); }
 
-template <int ACT, bool INT_EPI, int NK, int TJ>
+// INT_EPI: 0 every integer-epilogue term is zero; 1 zp_A = 0 (zero points of
+// the weights, or the row-VNNI formula with a caller's sum_W); 2 any zp_A (the
+// fixed-scale layers), whose K zp_W zp_A term is 64-bit; a.sumW is then the
+// sum the formula takes (the launcher passes the byte sums for an absent one).
+template <int ACT, int INT_EPI, int NK, int TJ>
 __global__ __launch_bounds__(kWideThreads, 1) void k_gemm_wide(RowsArgs a, int ntiles, int c0_mode) {
     using Cf = WideCfg<TJ>;
     constexpr int BM = Cf::BM, BN = Cf::BN, NL = Cf::NL, ROW = Cf::ROW, TI = Cf::TI;
@@ -266,7 +270,8 @@ __global__ __launch_bounds__(kWideThreads, 1) void k_gemm_wide(RowsArgs a, int n
                             : (INT_EPI && e == 3) ? static_cast<const void*>(a.sum_in ? a.sum_in + t.m0 : nullptr)
                             : (INT_EPI && e == 4) ? static_cast<const void*>(a.zpW ? a.zpW + t.n0 : nullptr)
                             : (INT_EPI && e == 5) ? static_cast<const void*>(c0_mode ? a.colsum_in + t.n0 : nullptr)
-                            : (INT_EPI && e == 6) ? static_cast<const void*>(c0_mode ? a.sumW + t.n0 : nullptr)
+                            : (INT_EPI == 1 && e == 6) ? static_cast<const void*>(c0_mode ? a.sumW + t.n0 : nullptr)
+                            : (INT_EPI == 2 && e == 6) ? static_cast<const void*>(a.sumW ? a.sumW + t.n0 : nullptr)
                             : nullptr;
             const int64_t len = (e == 2 || e == 3) ? 4 * rows : 4 * cols;
             const int32_t* dst = e == 0 ? reinterpret_cast<const int32_t*>(T.sw)
@@ -317,6 +322,10 @@ __global__ __launch_bounds__(kWideThreads, 1) void k_gemm_wide(RowsArgs a, int n
     struct ColC {
         float sw[TJ], bb[TJ];
         int32_t c0[TJ], c1[TJ];
+        // The 64-bit term, below 2^52 (K <= 2^10, |zp_A| <= 2^10): double
+        // holds its sum with a 32-bit integer exactly and rounds it to float
+        // as the 64-bit conversion does, without that one's branches.
+        double c2[INT_EPI == 2 ? TJ : 1];
     };
     auto col_consts = [&](const WideTables& T_, ColC& cc) {
 #pragma unroll
@@ -324,7 +333,16 @@ __global__ __launch_bounds__(kWideThreads, 1) void k_gemm_wide(RowsArgs a, int n
             const int col = 32 * TJ * wn + 32 * j + lr;
             cc.sw[j] = T_.sw[col];
             cc.bb[j] = T_.bias[col];
-            if constexpr (INT_EPI) {
+            if constexpr (INT_EPI == 2) {
+                // int_epi_consts's forms; c0_mode 0 is the batched one.
+                const uint32_t zpw = static_cast<uint32_t>(T_.zpw[col]), zpa = static_cast<uint32_t>(a.zp_A);
+                const uint32_t swr = static_cast<uint32_t>(T_.c0b[col]), cs = static_cast<uint32_t>(T_.c0a[col]);
+                cc.c1[j] = static_cast<int32_t>(0u - 2u * zpw);
+                cc.c0[j] = static_cast<int32_t>(c0_mode ? 128u * (cs - swr) - 2u * zpa * swr +
+                                                              3u * static_cast<uint32_t>(K) * zpa * zpw
+                                                        : 0u - zpa * swr);
+                cc.c2[j] = static_cast<double>(K * a.zp_A) * static_cast<double>(T_.zpw[col]);
+            } else if constexpr (INT_EPI == 1) {
                 cc.c1[j] = static_cast<int32_t>(0u - 2u * static_cast<uint32_t>(T_.zpw[col]));
                 cc.c0[j] = static_cast<int32_t>(128u * (static_cast<uint32_t>(T_.c0a[col]) -
                                                         static_cast<uint32_t>(T_.c0b[col])));
@@ -354,7 +372,11 @@ __global__ __launch_bounds__(kWideThreads, 1) void k_gemm_wide(RowsArgs a, int n
             for (int e = 0; e < 4; ++e) {
                 const int32_t d = acc[i][j][4 * q + e];
                 float tv;
-                if constexpr (INT_EPI)
+                if constexpr (INT_EPI == 2) {
+                    const int32_t t32 = static_cast<int32_t>(static_cast<uint32_t>(d) + static_cast<uint32_t>(cc.c0[j]) +
+                                                             static_cast<uint32_t>(cc.c1[j]) * static_cast<uint32_t>(sa_i[e]));
+                    tv = static_cast<float>(static_cast<double>(t32) + cc.c2[j]);
+                } else if constexpr (INT_EPI == 1)
                     tv = static_cast<float>(static_cast<int32_t>(static_cast<uint32_t>(d) + static_cast<uint32_t>(cc.c0[j]) +
                                                                  static_cast<uint32_t>(cc.c1[j]) * static_cast<uint32_t>(sa_i[e])));
                 else

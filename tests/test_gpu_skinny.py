@@ -80,7 +80,9 @@ def test_skinny_fp8(gpu, skinny, M, K, N):
 
 # Zero points whose product with K passes 2^31 make the 64-bit integer term.
 @pytest.mark.parametrize("M,K,N,zp_a,zp_w", [(300, 576, 68, 5, 6), (1025, 1024, 132, -7, 6), (4000, 512, 512, 3, 6),
-                                             (200, 4160, 64, 100, 6), (130, 2048, 60, 100000, 30000)])
+                                             (200, 4160, 64, 100, 6), (130, 2048, 60, 100000, 30000),
+                                             (700, 1024, 260, -1024, 1 << 24), (700, 1024, 260, 1025, 1 << 24),
+                                             (9000, 512, 1000, 0, 6), (66000, 512, 520, 7, 1 << 24)])
 @pytest.mark.parametrize("form", ["rows", "rows_sum", "batched"])
 def test_fixed_split(gpu, M, K, N, zp_a, zp_w, form):
     W = WL.uniform(860, (N, K), -0.125, 0.125)
