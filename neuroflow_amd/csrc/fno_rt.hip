@@ -1968,11 +1968,14 @@ hipError_t launch_post(const PostArgs& a, hipStream_t st) {
 }
 
 // The fused layer + tail: width 64, whole 32-token tiles (n a multiple of
-// 32), at least two tiles per CU, the runtime's activations (ReLU, GELU) and
-// next-input fake-quants (off, per tensor), and the layer of 64 x 64.
+// 32), the runtime's activations (ReLU, GELU) and next-input fake-quants (off,
+// per tensor), and the layer of 64 x 64.  At any number of tiles: also where
+// few tiles leave most CUs idle, one launch is shorter than two (FNO1d of 4
+// layers, 1 x 256 of width 64 INT8 91 -> 86 us, 8 x 1024 127 -> 107, 10 x 1024
+// fp32 164 -> 126; FNO2d 3 x 64 x 64 of width 32 156 -> 114).
 bool layer_tail_ok(const PostArgs& p, int in_features, int out_features) {
     return !path_flag(kernel_path().no_layer_tail) && p.w == 64 && in_features == 64 && out_features == 64 &&
-           p.n > 0 && p.n % 32 == 0 && tile_count(p.samples, p.n, p.w, 32) >= 2 * static_cast<int64_t>(num_cus()) &&
+           p.n > 0 && p.n % 32 == 0 &&
            (p.act == RT_ACT_RELU || p.act == RT_ACT_GELU) && (p.fq_next.on == 0 || p.fq_next.on == 1) &&
            p.kind >= 0 && p.kind <= 3 && aligned(p.h, 16);
 }
@@ -2041,13 +2044,12 @@ hipError_t launch_linear_tail(const PostArgs& a, const float* W, const float* b,
 }
 
 // The projection head in one launch: proj_q 64 -> 64 and proj_out 64 -> 1,
-// whole 32-token tiles, at least two tiles per CU, the fake-quant forms off /
-// per tensor / log2 snap, 16-byte aligned h rows and proj_q weight.
+// whole 32-token tiles, the fake-quant forms off / per tensor / log2 snap, 16-byte aligned h rows and proj_q weight.
 bool proj_tail_ok(const ProjArgs& p) {
     if (p.w != 64) return proj_tail_w_ok(p);
     const auto fq_ok = [](const FakeQuant& f) { return f.on == 0 || f.on == 1 || f.on == 3; };
     return !path_flag(kernel_path().no_layer_tail) && p.w == 64 && p.out_ch == 1 && p.n > 0 && p.n % 32 == 0 &&
-           p.rows_in >= p.n && tile_count(p.samples, p.n, 64, 32) >= 2 * static_cast<int64_t>(num_cus()) &&
+           p.rows_in >= p.n &&
            fq_ok(p.fq_q) && fq_ok(p.fq_o) && (p.act == RT_ACT_NONE || p.act == RT_ACT_RELU || p.act == RT_ACT_GELU) &&
            aligned(p.h, 16) && aligned(p.Wq, 16);
 }

@@ -190,13 +190,11 @@ __global__ __launch_bounds__(256) void k_proj_tail_w(ProjArgs a) {
 
 // Widths with an instantiation: the multiples of 8 below 64 and 20 (others
 // keep the separate launches).  The rest of the conditions are the width-64
-// forms': whole 32-token tiles, at least two per CU, the runtime's
-// activations and fake-quants.
+// forms': whole 32-token tiles, the runtime's activations and fake-quants.
 static bool width_ok(int w) { return w == 16 || w == 20 || w == 24 || w == 32 || w == 40 || w == 48; }
 
 bool linear_tail_w_ok(const PostArgs& p, const float* W) {
     return !path_flag(kernel_path().no_layer_tail) && width_ok(p.w) && p.n > 0 && p.n % 32 == 0 &&
-           tile_count(p.samples, p.n, p.w, 32) >= 2 * static_cast<int64_t>(num_cus()) &&
            (p.act == RT_ACT_RELU || p.act == RT_ACT_GELU) && (p.fq_next.on == 0 || p.fq_next.on == 1) &&
            (p.kind == 0 || p.kind == 1 || p.kind == 3) && aligned(p.h, 16) && aligned(W, 16);
 }
@@ -204,7 +202,7 @@ bool linear_tail_w_ok(const PostArgs& p, const float* W) {
 bool proj_tail_w_ok(const ProjArgs& p) {
     const auto fq_ok = [](const FakeQuant& f) { return f.on == 0 || f.on == 1 || f.on == 3; };
     return !path_flag(kernel_path().no_layer_tail) && width_ok(p.w) && p.out_ch == 1 && p.n > 0 && p.n % 32 == 0 &&
-           p.rows_in >= p.n && tile_count(p.samples, p.n, p.w, 32) >= 2 * static_cast<int64_t>(num_cus()) &&
+           p.rows_in >= p.n &&
            fq_ok(p.fq_q) && fq_ok(p.fq_o) && (p.act == RT_ACT_RELU || p.act == RT_ACT_GELU) && aligned(p.h, 16) &&
            aligned(p.Wq, 16);
 }

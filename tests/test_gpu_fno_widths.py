@@ -38,8 +38,10 @@ def _run(tmp_path, ir, x, out_ch, flag=0, int8=False):
         _lib.check(L.nflow_debug_set_kernel_path(b"no_layer_tail", prev.value, None), "path")
 
 
-# 512 whole 32-token tiles: the smallest batch the fused forms take (two per CU).
-FUSED = [(16, 1024, 1, 1, w, 6, 2, 1, relu, kinds, False)
+# 512 whole 32-token tiles (several per block), then one and a few tiles.
+FUSED = [(1, 32, 1, 1, 64, 6, 2, 1, False, ["tensor"], True), (2, 64, 1, 1, 64, 6, 2, 1, True, ["token", "tensor"], False),
+         (1, 32, 1, 1, 20, 6, 2, 1, False, ["tensor"], False), (3, 32, 1, 1, 48, 6, 2, 1, False, ["fp8"], False)] + \
+        [(16, 1024, 1, 1, w, 6, 2, 1, relu, kinds, False)
          for w, relu, kinds in [(16, False, ["tensor"]), (20, True, None), (20, False, ["fp8"]), (24, False, ["tensor"]),
                                 (32, True, ["fp8", "tensor"]), (32, False, None), (40, False, ["tensor", "fp8"]),
                                 (48, False, ["tensor"]), (48, True, ["fp8"])]]
@@ -50,7 +52,7 @@ def test_fused_widths_fno1d(gpu, tmp_path, case):
     ir, x, m = T1._model(case)
     want = OF.forward(m, x)
     for flag in (0, 1):
-        y = _run(tmp_path, ir, x, 1, flag)
+        y = _run(tmp_path, ir, x, 1, flag, case[10])
         assert np.array_equal(T1._bits(y), T1._bits(want)), (flag, int((T1._bits(y) != T1._bits(want)).sum()))
 
 
