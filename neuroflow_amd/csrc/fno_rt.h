@@ -200,10 +200,12 @@ struct ProjArgs {
 };
 bool proj_tail_ok(const ProjArgs& p);
 hipError_t launch_proj_tail(const ProjArgs& a, hipStream_t st);
-// The widths other than 64 (fno_tail.hip); linear_tail_ok, proj_tail_ok and
-// their launchers call these.
+// The widths other than 64 (fno_tail.hip); layer_tail_ok, linear_tail_ok,
+// proj_tail_ok and their launchers call these.
 bool linear_tail_w_ok(const PostArgs& p, const float* W);
 hipError_t launch_linear_tail_w(const PostArgs& a, const float* W, const float* b, hipStream_t st);
+bool layer_tail_w_ok(const PostArgs& p, int in_features, int out_features);
+hipError_t launch_layer_tail_w(const LayerTailArgs& a, hipStream_t st);
 bool proj_tail_w_ok(const ProjArgs& p);
 hipError_t launch_proj_tail_w(const ProjArgs& a, hipStream_t st);
 // The device arrays of an INT8 layer handle into a (layer.cpp): false for

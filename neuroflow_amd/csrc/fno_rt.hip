@@ -1974,6 +1974,7 @@ hipError_t launch_post(const PostArgs& a, hipStream_t st) {
 // layers, 1 x 256 of width 64 INT8 91 -> 86 us, 8 x 1024 127 -> 107, 10 x 1024
 // fp32 164 -> 126; FNO2d 3 x 64 x 64 of width 32 156 -> 114).
 bool layer_tail_ok(const PostArgs& p, int in_features, int out_features) {
+    if (p.w != 64) return layer_tail_w_ok(p, in_features, out_features);
     return !path_flag(kernel_path().no_layer_tail) && p.w == 64 && in_features == 64 && out_features == 64 &&
            p.n > 0 && p.n % 32 == 0 &&
            (p.act == RT_ACT_RELU || p.act == RT_ACT_GELU) && (p.fq_next.on == 0 || p.fq_next.on == 1) &&
@@ -2002,6 +2003,7 @@ static void launch_layer_tail_act(const LayerTailArgs& a, unsigned grid, hipStre
 
 hipError_t launch_layer_tail(const LayerTailArgs& a, hipStream_t st) {
     if (a.p.samples <= 0) return hipSuccess;
+    if (a.p.w != 64) return launch_layer_tail_w(a, st);
     const unsigned grid = grid_for(tile_count(a.p.samples, a.p.n, a.p.w, 32), 1, 8);
     switch (a.p.kind) {
         case 1: launch_layer_tail_act<1>(a, grid, st); break;

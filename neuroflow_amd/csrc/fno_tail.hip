@@ -1,5 +1,5 @@
-// fno_tail.hip -- the FNO runtime's fp32 local linear with the layer tail,
-// and the projection head, each in one launch, for widths other than 64
+// fno_tail.hip -- the FNO runtime's local linear (fp32 or INT8) with the layer
+// tail, and the projection head, each in one launch, for widths other than 64
 // (fno_rt.hip holds the width-64 forms).
 //
 // What bounds them: the ordered fp32 sums (one multiply and one add per term,
@@ -124,6 +124,100 @@ __global__ __launch_bounds__(256) void k_linear_tail_w(PostArgs a, const float* 
     }
 }
 
+// The INT8 local linear (LinearForwardBatched + bias with the layer's
+// per-tensor scale, as fno.cpp:529-536 runs it) and the tail on the same
+// tiles: the h tile becomes codes in LDS, four per dword, a thread holds its
+// channel's W weight codes in W / 4 registers, and an output's product is W / 4
+// v_dot4 (exact in int32; at these widths fewer instructions than the moves an
+// MFMA's operand layouts would take).  As two launches (the fixed-scale layer
+// and the tail) an FNO1d of 4 layers, 256 x 1024 of width 32, ran 484 us; 310
+// with this kernel (60 x 1024: 232 -> 149).
+template <int W, int KIND, int ACT, int FQN>
+__global__ __launch_bounds__(256) void k_layer_tail_w(LayerTailArgs la, int int_epi) {
+    using S = TailShape<W>;
+    constexpr int KQ = W / 4, CS = KQ + 1;           // code dwords per token, row stride
+    const PostArgs& a = la.p;
+    __shared__ float tx1[W][S::TT + 1];
+    __shared__ uint32_t codes[S::TT * CS];
+    __shared__ float thr_x2[16], thr_next[16];
+    const int n = a.n;                  // n % 32 == 0 (layer_tail_w_ok)
+    if (threadIdx.x < 15) thr_x2[threadIdx.x] = a.thr[threadIdx.x];
+    stage_steps(thr_next, a.fq_next.thr);
+    const ScaleInv inv_x2 = scale_inv(a.scale), inv_next = scale_inv(a.fq_next.scale);
+    const float fixed_inv = 1.0f / la.sA;
+    const bool fixed_fast = la.sA >= 0x1p-120f && la.sA <= 0x1p120f;
+    const int tid = threadIdx.x;
+    const int cm = tid / S::TT, tm = tid % S::TT;            // channel-major: channel, token
+    const int tk = tid / W, ck = tid % W;                    // token-major: token, channel
+    const bool live = tid < S::RP * W;
+    uint32_t wq[KQ];
+    int32_t sfull = 0;
+#pragma unroll
+    for (int q = 0; q < KQ; ++q) {
+        wq[q] = reinterpret_cast<const uint32_t*>(la.W + ck * W)[q];
+        sfull = sum_bytes_i8(wq[q], sfull);
+    }
+    const IntEpi epi = int_epi_consts(F_BATCHED, W, la.zpA, la.zpW ? la.zpW[ck] : 0, la.sumW ? la.sumW[ck] : 0,
+                                      la.sumW != nullptr, sfull, sfull);
+    const float sw = la.sW[ck], bj = la.bias ? la.bias[ck] : 0.0f;
+    const int64_t o1 = static_cast<int64_t>(cm) * n + tm, d1 = static_cast<int64_t>(8) * n;
+    Tile tl;
+    for (int64_t id = blockIdx.x; tile_of<S::TT>(id, a.samples, n, W, tl); id += gridDim.x) {
+        const int64_t cb = tl.s * W * static_cast<int64_t>(n) + tl.t0 + o1;
+        const int64_t tb = (tl.s * n + tl.t0) * W;
+        v4f hv[S::HV];
+#pragma unroll
+        for (int q = 0; q < S::HV; ++q)
+            if (S::NV % 256 == 0 || tid + 256 * q < S::NV) hv[q] = *reinterpret_cast<const v4f*>(a.h + tb + 4 * (tid + 256 * q));
+        float xv[S::XV];
+#pragma unroll
+        for (int q = 0; q < S::XV; ++q)
+            if (W % 8 == 0 || cm + 8 * q < W) xv[q] = a.x1c[cb + q * d1];
+#pragma unroll
+        for (int q = 0; q < S::XV; ++q)
+            if (W % 8 == 0 || cm + 8 * q < W) tx1[cm + 8 * q][tm] = xv[q];
+#pragma unroll
+        for (int q = 0; q < S::HV; ++q) {
+            const int i = tid + 256 * q;
+            if (S::NV % 256 == 0 || i < S::NV)
+                codes[(i / KQ) * CS + i % KQ] = quant_i8_fixed4(hv[q], la.sA, fixed_inv, la.zpA, fixed_fast);
+        }
+        __syncthreads();
+        float v[S::PER];
+#pragma unroll
+        for (int q = 0; q < S::PER; ++q) {
+            const int t = tk + S::RP * q;
+            if (S::TT % S::RP != 0 && t >= S::TT) continue;
+            if (!live) continue;
+            const uint32_t* cr = codes + t * CS;
+            int32_t D = 0, SA = 0;
+#pragma unroll
+            for (int k = 0; k < KQ; ++k) D = __builtin_amdgcn_sdot4(static_cast<int>(cr[k]), static_cast<int>(wq[k]), D, false);
+            float tv;
+            if (int_epi) {
+#pragma unroll
+                for (int k = 0; k < KQ; ++k) SA = sum_bytes_i8(cr[k], SA);
+                tv = int_epi_value(epi, D, SA);
+            } else {
+                tv = static_cast<float>(D);
+            }
+            const float x2 = dequant_bias(sw, la.sA, tv, bj);
+            v[q] = post_element<KIND, ACT, FQN>(tx1[ck][t], x2, a, inv_x2, inv_next, thr_x2, thr_next, 0.0f, 0.0f);
+            tx1[ck][t] = v[q];
+        }
+#pragma unroll
+        for (int q = 0; q < S::PER; ++q) {
+            const int t = tk + S::RP * q;
+            if (live && (S::TT % S::RP == 0 || t < S::TT)) a.h[tb + t * W + ck] = v[q];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < S::XV; ++q)
+            if (W % 8 == 0 || cm + 8 * q < W) a.hc[cb + q * d1] = tx1[cm + 8 * q][tm];
+        __syncthreads();
+    }
+}
+
 // The projection head (fno.cpp:662-698, :966-993): proj_q W -> W, its
 // fake-quant FQQ and the activation, then proj_out W -> 1 (32 threads, one
 // token each, the W activations in order) and its fake-quant.
@@ -199,6 +293,10 @@ bool linear_tail_w_ok(const PostArgs& p, const float* W) {
            (p.kind == 0 || p.kind == 1 || p.kind == 3) && aligned(p.h, 16) && aligned(W, 16);
 }
 
+bool layer_tail_w_ok(const PostArgs& p, int in_features, int out_features) {
+    return in_features == p.w && out_features == p.w && linear_tail_w_ok(p, nullptr);
+}
+
 bool proj_tail_w_ok(const ProjArgs& p) {
     const auto fq_ok = [](const FakeQuant& f) { return f.on == 0 || f.on == 1 || f.on == 3; };
     return !path_flag(kernel_path().no_layer_tail) && width_ok(p.w) && p.out_ch == 1 && p.n > 0 && p.n % 32 == 0 &&
@@ -236,6 +334,42 @@ hipError_t launch_linear_tail_w(const PostArgs& a, const float* Wl, const float*
         case 32: launch_lt<32>(a, Wl, b, st); break;
         case 40: launch_lt<40>(a, Wl, b, st); break;
         default: launch_lt<48>(a, Wl, b, st); break;
+    }
+    return hipGetLastError();
+}
+
+template <int W, int KIND, int ACT>
+static void launch_layt_fqn(const LayerTailArgs& a, int int_epi, unsigned grid, hipStream_t st) {
+    if (a.p.fq_next.on == 1)
+        hipLaunchKernelGGL((k_layer_tail_w<W, KIND, ACT, 1>), dim3(grid), dim3(256), 0, st, a, int_epi);
+    else
+        hipLaunchKernelGGL((k_layer_tail_w<W, KIND, ACT, 0>), dim3(grid), dim3(256), 0, st, a, int_epi);
+}
+
+template <int W, int KIND>
+static void launch_layt_act(const LayerTailArgs& a, int int_epi, unsigned grid, hipStream_t st) {
+    if (a.p.act == RT_ACT_GELU) launch_layt_fqn<W, KIND, RT_ACT_GELU>(a, int_epi, grid, st);
+    else launch_layt_fqn<W, KIND, RT_ACT_RELU>(a, int_epi, grid, st);
+}
+
+template <int W>
+static void launch_layt(const LayerTailArgs& a, hipStream_t st) {
+    const unsigned grid = grid_for(tile_count(a.p.samples, a.p.n, a.p.w, 32), 1, 8);
+    const int int_epi = a.zpA != 0 || a.zpW;
+    if (a.p.kind == 1) launch_layt_act<W, 1>(a, int_epi, grid, st);
+    else if (a.p.kind == 3) launch_layt_act<W, 3>(a, int_epi, grid, st);
+    else launch_layt_act<W, 0>(a, int_epi, grid, st);
+}
+
+hipError_t launch_layer_tail_w(const LayerTailArgs& a, hipStream_t st) {
+    if (a.p.samples <= 0) return hipSuccess;
+    switch (a.p.w) {
+        case 16: launch_layt<16>(a, st); break;
+        case 20: launch_layt<20>(a, st); break;
+        case 24: launch_layt<24>(a, st); break;
+        case 32: launch_layt<32>(a, st); break;
+        case 40: launch_layt<40>(a, st); break;
+        default: launch_layt<48>(a, st); break;
     }
     return hipGetLastError();
 }

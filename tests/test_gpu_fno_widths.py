@@ -40,6 +40,9 @@ def _run(tmp_path, ir, x, out_ch, flag=0, int8=False):
 
 # 512 whole 32-token tiles (several per block), then one and a few tiles.
 FUSED = [(1, 32, 1, 1, 64, 6, 2, 1, False, ["tensor"], True), (2, 64, 1, 1, 64, 6, 2, 1, True, ["token", "tensor"], False),
+         (16, 1024, 1, 1, 32, 6, 3, 1, False, ["tensor"], True), (3, 64, 1, 1, 48, 6, 3, 1, True, ["tensor", "fp8", "tensor"], True),
+         (2, 32, 1, 1, 20, 6, 3, 1, False, ["fp8", "tensor"], True), (5, 32, 1, 1, 16, 6, 2, 1, False, ["tensor"], True),
+         (2, 64, 1, 1, 24, 6, 2, 1, False, ["tensor"], True), (2, 64, 1, 1, 40, 6, 2, 1, False, ["tensor"], True),
          (1, 32, 1, 1, 20, 6, 2, 1, False, ["tensor"], False), (3, 32, 1, 1, 48, 6, 2, 1, False, ["fp8"], False)] + \
         [(16, 1024, 1, 1, w, 6, 2, 1, relu, kinds, False)
          for w, relu, kinds in [(16, False, ["tensor"]), (20, True, None), (20, False, ["fp8"]), (24, False, ["tensor"]),
