@@ -619,6 +619,12 @@ struct Scratch {
     Scratch& operator=(const Scratch&) = delete;
 };
 
+// Whether a graph capture is recording stream st.
+static bool stream_capturing(hipStream_t st) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
+}
+
 static int kb_dot_for(int formula, int K) {
     if (formula == F_ROW_VNNI) return K / 64;   // int8_gemm.cpp:366: vec_end = K - K % 64
     return (K + 63) / 64;
@@ -738,6 +744,11 @@ static int int8_fixed_path(const nflow_int8_linear_params* p, int64_t rows, cons
         const bool want_colsum = gemm_needs_colsum(a);
         const size_t codes16 = ((static_cast<size_t>(rows) * a.K + 15) / 16) * 16;
         Scratch ws(codes16 + (2 * static_cast<size_t>(rows) + (want_colsum ? a.N : 0)) * sizeof(int32_t), st);
+        if (ws.err != hipSuccess && use_token_gemm(a)) {
+            (void)hipGetLastError();
+            launch_token_i8_fixed(a, st);
+            return check_launch(what);
+        }
         if (ws.err != hipSuccess) return set_error(NFLOW_INTERNAL, std::string(what) + ": workspace allocation failed");
         uint8_t* q = static_cast<uint8_t*>(ws.p);
         float* sc = reinterpret_cast<float*>(q + codes16);
@@ -1025,7 +1036,11 @@ static int int8_per_token(const nflow_int8_linear_params* p, int64_t M, const fl
         launch_skinny_i8(a, act_x2, st);
         return finish();
     }
-    if (!refused && use_token_gemm(a) && !(wide && split_faster(a))) {
+    // The split form allocates: not where its codes exceed the no-allocation
+    // scratch, nor for a capture that the one-pass kernel can serve.
+    const bool one_pass = use_token_gemm(a);
+    if (!refused && one_pass && !(wide && split_faster(a) && !(fixed && noalloc_need(a, wide) > fixed->cap) &&
+                                  !(a.K <= 512 && !fixed && stream_capturing(st)))) {
         launch_token_i8(a, act_x2, st);
         return finish();
     }
@@ -1069,6 +1084,11 @@ static int int8_per_token(const nflow_int8_linear_params* p, int64_t M, const fl
         return finish();
     }
     Scratch ws(codes + 16 + static_cast<size_t>(M) * sizeof(float) + n_sums * sizeof(int32_t), st);
+    if (ws.err != hipSuccess && one_pass) {
+        (void)hipGetLastError();
+        launch_token_i8(a, act_x2, st);
+        return finish();
+    }
     if (ws.err != hipSuccess) return set_error(NFLOW_INTERNAL, "linear_forward_per_token: workspace allocation failed");
     uint8_t* q = static_cast<uint8_t*>(ws.p);
     float* sc = reinterpret_cast<float*>(q + codes16);
@@ -1288,6 +1308,11 @@ static int fp8_per_token(const nflow_fp8_linear_params* p, int64_t M, const floa
     }
     const size_t codes = static_cast<size_t>(M) * a.K;
     Scratch ws(codes + 16 + static_cast<size_t>(M) * sizeof(float), st);
+    if (ws.err != hipSuccess && use_token_gemm(a)) {
+        (void)hipGetLastError();
+        launch_token_fp8(a, act_x2, st);
+        return finish();
+    }
     if (ws.err != hipSuccess) return set_error(NFLOW_INTERNAL, "fp8_linear_forward_per_token: workspace allocation failed");
     uint8_t* q = static_cast<uint8_t*>(ws.p);
     float* sc = reinterpret_cast<float*>(q + ((codes + 15) / 16) * 16);
@@ -1443,18 +1468,14 @@ static int chain_words(ChainState* cs, int64_t M, hipStream_t st) {
     return NFLOW_OK;
 }
 
-// The chain entry points under graph capture: refused before any
-// allocation or launch.  The fused kernel's row-maxima words would be
-// allocated and cleared inside the graph and a replay would reuse its
-// launch's epoch (an earlier replay's words reading as fresh); the
-// layer-by-layer route allocates its buffers inside the graph, and a graph
-// captured that way (both entry points, 20000 rows) took an illegal memory
-// access on its first replay, for a reason not found in this library.
-static bool stream_capturing(hipStream_t st) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
-}
-
+// The chain entry points refuse a capturing stream before any allocation or
+// launch: the fused kernel's row-maxima words would be allocated and cleared
+// inside the graph and a replay would reuse its launch's epoch (an earlier
+// replay's words reading as fresh); the layer-by-layer route allocates its
+// buffers inside the graph, and a graph captured that way (both entry
+// points, 20000 rows) took an illegal memory access on its first replay, for
+// a reason not found in this library.
+//
 // Whether calls on stream st may use the fused 8-bit-output kernel: not on
 // the per-thread default stream, whose one handle names a different stream
 // in each host thread, so concurrent launches would share the row-maxima

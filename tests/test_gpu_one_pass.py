@@ -138,3 +138,20 @@ def test_fp8(gpu, tile_rows, M, K, N):
     bound = (K + 3) * 2.0 ** -24 * (terms + np.abs(b)[None, :]) + 1e-38
     assert np.all(np.abs(got[fin].astype(np.float64) - want[fin]) <= bound)
     assert _guards_kept(buf, M, N, off)
+
+
+def test_noalloc_large_codes_keep_the_one_pass_kernel(gpu):
+    """K = 512 with a wide N takes quantise + GEMM where that is faster, but the
+    no-allocation entry point, whose scratch cannot hold 160000 rows of codes,
+    serves it all the same (it never needed scratch at K = 512)."""
+    M, K, N = 160000, 512, 576
+    q, s, _, _, b = _int8(N, K, 870)
+    x = torch.from_numpy(WL.normal(873, (1000, K))).cuda().repeat(M // 1000, 1)
+    p = Q.Int8LinearParams(_cu(q, 0), _cu(s, 0), None, _cu(b, 0))
+    ps = p.c_struct()
+    out = torch.empty(M, N, device="cuda")
+    rc = _lib.lib().nflow_int8_linear_forward_per_token_noalloc(ctypes.byref(ps), M, x.data_ptr(), out.data_ptr(), None,
+                                                                0, torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "noalloc")
+    want = Q.linear_forward_per_token(p, x, "none")
+    assert torch.equal(out.view(torch.int32), want.view(torch.int32))
