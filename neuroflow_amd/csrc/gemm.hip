@@ -6,8 +6,9 @@
 namespace nfq {
 
 bool gemm_ok(const RowsArgs& a) {
-    // K <= 65536 keeps a 256-row tile's byte count inside the 32-bit buffer range.
-    return a.K % 64 == 0 && a.K >= 128 && a.K <= 65536 && a.N % 4 == 0 && a.kb_dot * 64 >= a.K &&
+    // K <= 65536 keeps a 256-row tile's byte count inside the 32-bit buffer
+    // range, N <= 2^24 a 16-row output strip's.
+    return a.K % 64 == 0 && a.K >= 128 && a.K <= 65536 && a.N % 4 == 0 && a.N <= (1 << 24) && a.kb_dot * 64 >= a.K &&
            aligned(a.Aq, 16) && aligned(a.W, 16) && aligned(a.C, 16);
 }
 

@@ -70,6 +70,15 @@ inline bool aligned(const void* p, uintptr_t a) {
     return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0;
 }
 
+// Whether the output of a layer on fp32 input overlaps that input.  A square
+// layer may run in place: every kernel reads a row tile before it writes it,
+// as long as one block alone holds the tile.
+inline bool in_place(const RowsArgs& a) {
+    const char* x = reinterpret_cast<const char*>(a.A);
+    const char* y = static_cast<const char*>(a.C);
+    return x && y && x < y + 4 * a.M * a.N && y < x + 4 * a.M * a.K;
+}
+
 // Row-tile kernel eligibility for the given input mode.  On fp32 input it
 // serves K, N <= 64, its weights in registers for the whole launch; the
 // one-pass kernel takes the others (with two K blocks, 100000 x 128 -> 64, the

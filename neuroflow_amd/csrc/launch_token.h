@@ -14,8 +14,9 @@ static void launch_token_k(const RowsArgs& a, hipStream_t st) {
     const int64_t tiles = (a.M + 16 * RT - 1) / (16 * RT);
     const int64_t slots = static_cast<int64_t>(num_cus()) * per_cu;
     // Fewer row tiles than resident blocks: the column chunks of a tile are
-    // shared out over several blocks, each quantising the tile for itself.
-    const int64_t chunks = (a.N + 64 * CT - 1) / (64 * CT);
+    // shared out over several blocks, each quantising the tile for itself (not
+    // in place: one of them could write rows that another has yet to read).
+    const int64_t chunks = in_place(a) ? 1 : (a.N + 64 * CT - 1) / (64 * CT);
     const int64_t share = std::max<int64_t>(1, std::min<int64_t>(chunks, slots / tiles));
     const int64_t grid = std::min<int64_t>(tiles * share, slots);
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(grid)), dim3(256), 0, st, a, static_cast<int>(share));

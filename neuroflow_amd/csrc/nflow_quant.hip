@@ -656,7 +656,7 @@ static bool use_token_gemm(const RowsArgs& a) {
 // (128) 13 / 19, 128 rows (1024) 67 / 21.
 static bool use_skinny(const RowsArgs& a) {
     const int f = kernel_path().skinny.load(std::memory_order_relaxed);
-    if (f == 2 || !skinny_ok(a)) return false;
+    if (f == 2 || !skinny_ok(a) || in_place(a)) return false;   // its blocks share rows
     if (f == 1) return true;
     const int64_t blocks = ((a.M + 15) / 16) * ((static_cast<int64_t>(a.N) + 15) / 16);
     const int64_t cus = num_cus();

@@ -155,3 +155,31 @@ def test_noalloc_large_codes_keep_the_one_pass_kernel(gpu):
     _lib.check(rc, "noalloc")
     want = Q.linear_forward_per_token(p, x, "none")
     assert torch.equal(out.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("M,K", [(1, 64), (8, 200), (16, 1024), (300, 200), (300, 512), (5000, 256), (70, 1024), (33, 96)])
+@pytest.mark.parametrize("fmt", ["int8", "fp8", "fixed"])
+def test_square_layer_in_place(gpu, M, K, fmt):
+    """out = the input tensor: the same bits as out of place (a tile's columns
+    are then not shared over blocks, and rows not over the few-row kernel's)."""
+    A = WL.normal(880, (M, K))
+    if fmt == "fp8":
+        qw, sw = O.quantise_weight_fp8(WL.uniform(881, (K, K), -0.125, 0.125))
+        p = Q.Fp8LinearParams(_cu(qw, 0), _cu(sw, 0))
+        fn, args = _lib.lib().nflow_fp8_linear_forward_per_token, (None, 1)
+    else:
+        q, s, zps, sw, b = _int8(K, K, 882)
+        p = Q.Int8LinearParams(_cu(q, 0), _cu(s, 0), _cu(zps, 0), _cu(b, 0), 0.02, 3)
+        fn, args = ((_lib.lib().nflow_int8_linear_forward_per_token, (None, 1)) if fmt == "int8"
+                    else (_lib.lib().nflow_int8_linear_forward_rows, ()))
+    ps, st = p.c_struct(), torch.cuda.current_stream().cuda_stream
+    x = _cu(A, 0)
+    out = torch.empty(M, K, device="cuda")
+    _lib.check(fn(ctypes.byref(ps), M, x.data_ptr(), out.data_ptr(), *args, st), "layer")
+    for _ in range(3):
+        y = _cu(A, 0)
+        _lib.check(fn(ctypes.byref(ps), M, y.data_ptr(), y.data_ptr(), *args, st), "in place")
+        if fmt == "fp8":     # another kernel may sum in another order
+            assert torch.allclose(y, out, rtol=1e-5, atol=1e-5)
+        else:
+            assert torch.equal(y.view(torch.int32), out.view(torch.int32))
