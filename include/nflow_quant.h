@@ -180,18 +180,25 @@ int nflow_int8_linear_forward_per_token(const nflow_int8_linear_params* p, int64
 /* nflow_int8_linear_forward_per_token that allocates nothing.  No
  * counterpart in the reference: it is for callers that cannot allocate --
  * code under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc.  Same arguments and results, bit for bit.  The
- * shapes the one-launch kernels do not take (e.g. K = 1024: per-token
- * quantise into codes, then the tiled GEMM) keep their codes, scales and
- * byte sums in a static device array of NFLOW_NOALLOC_SCRATCH_BYTES held by
- * each GPU the library runs on until the process ends, instead of a
- * stream-ordered allocation.  Workspace = M*K rounded up to 16, + 4M
- * (scales, unless scale_A_out is given), + 4M (row code sums, with zero
- * points), + 4N (weight-row sums, with a caller's sum_W); a call needing more
- * than the array returns NFLOW_INVALID_ARG before anything is launched.
- * Every call on one GPU shares that array and keeps nothing in it between
- * calls.  Host threads are safe when their calls share a stream: a
- * per-device lock is held from the array's lookup until the call's last
+ * hipMalloc.  Same arguments and results, bit for bit.
+ *
+ * Two kinds of shapes, at buffers aligned to 16 bytes, never use any scratch,
+ * whatever M: K = 128, 256 or 512 with N a multiple of 64; and K <= 256 that is a
+ * multiple of 4 but not of 64 (or K = 64), with N a multiple of 4.  Calls on
+ * them are independent of every other call, on any stream.
+ *
+ * Every other shape may run as a per-token quantise into codes and a tiled
+ * GEMM that keep codes, scales and byte sums in a static device array of
+ * NFLOW_NOALLOC_SCRATCH_BYTES held by each GPU the library runs on until
+ * the process ends, instead of a stream-ordered allocation.  Workspace = M*K
+ * rounded up to 16, + 4M (scales, unless scale_A_out is given), + 4M (row code
+ * sums, with zero points), + 4N (weight-row sums, with a caller's sum_W); a
+ * call whose workspace would be larger than the array returns
+ * NFLOW_INVALID_ARG before anything is launched, also where a kernel that
+ * needs none would have run it (the limit does not depend on which kernel the
+ * library prefers).  Those calls on one GPU share the array and keep nothing
+ * in it between calls.  Host threads are safe when their calls share a stream:
+ * a per-device lock is held from the array's lookup until the call's last
  * launch, so their launches do not interleave.  Calls on different streams
  * that the caller does not order race on the device. */
 int nflow_int8_linear_forward_per_token_noalloc(const nflow_int8_linear_params* p, int64_t M,

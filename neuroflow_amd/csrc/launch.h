@@ -115,6 +115,12 @@ void launch_rows64_fixed(const RowsArgs& a, hipStream_t st);
 // The one-pass layer for K <= 1024 (token_*.hip): quantise into LDS, then the
 // whole N range.
 bool token_gemm_ok(const RowsArgs& a);
+// Whole K blocks and column strips at 16-byte aligned buffers, no masks
+// needed (RAG = false), and K small enough for 64-row tiles.
+inline bool token_whole(const RowsArgs& a) {
+    return (a.K == 128 || a.K == 256 || a.K == 512) && a.N % 64 == 0 && aligned(a.A, 16) && aligned(a.C, 16) &&
+           aligned(a.W, 16);
+}
 // Whether it takes tiles of 16 rows (and 128-column chunks) instead of 64.
 bool token_small_tiles(const RowsArgs& a);
 void launch_token_i8(const RowsArgs& a, int act, hipStream_t st);

@@ -44,9 +44,7 @@ template <int FMT>
 static void launch_token_fmt(const RowsArgs& a, int act, hipStream_t st) {
     if (token_small_tiles(a)) return launch_token_rag<FMT, 2, 1>(a, act, st);
     if (a.N <= 128) return launch_token_rag<FMT, 2, 4>(a, act, st);
-    const bool whole = (a.K == 128 || a.K == 256 || a.K == 512) && a.N % 64 == 0 && aligned(a.A, 16) &&
-                       aligned(a.C, 16) && aligned(a.W, 16);
-    if (!whole) return launch_token_rag<FMT, 4, 4>(a, act, st);
+    if (!token_whole(a)) return launch_token_rag<FMT, 4, 4>(a, act, st);
     if (a.K == 128) launch_token_act<2, FMT, 4, 4, false>(a, act, st);
     else if (a.K == 256) launch_token_act<4, FMT, 4, 4, false>(a, act, st);
     else launch_token_act<8, FMT, 4, 4, false>(a, act, st);

@@ -974,18 +974,20 @@ static size_t noalloc_need(const RowsArgs& a, bool wide) {
     return codes16 + (a.scale_out ? 0 : static_cast<size_t>(a.M) * sizeof(float)) +
            split_sums(a, wide) * sizeof(int32_t);
 }
-// Shapes the no-allocation entry point documents as too large for its
-// scratch: those whose codes the split path holds there, also where the
-// one-pass kernel, which needs none, runs them (K = 128, 256 and 512 with N a
-// multiple of 64, and aligned K <= 256 the tiled GEMM cannot take, are never
-// refused).
-static bool noalloc_refuses(const RowsArgs& a, bool wide, size_t cap) {
-    const bool one_pass = (a.K == 128 || a.K == 256 || a.K == 512) && a.N % 64 == 0 && aligned(a.A, 16) &&
-                          aligned(a.C, 16) && aligned(a.W, 16);
+// Shapes the no-allocation entry point documents as never touching its
+// scratch: K = 128, 256 and 512 with N a multiple of 64, and K <= 256 the tiled
+// GEMM cannot take (K, N multiples of 4), both at aligned buffers.  Calls on
+// them are independent of every other call, on any stream.
+static bool noalloc_scratch_free(const RowsArgs& a, bool wide) {
     const bool narrow = !wide && a.K <= 256 && a.K % 4 == 0 && a.N % 4 == 0 && aligned(a.A, 16) &&
                         aligned(a.W, 4) && aligned(a.C, 16);
-    if (one_pass || narrow) return false;
-    return noalloc_need(a, wide) > cap;
+    return token_whole(a) || narrow;
+}
+// Shapes it documents as too large for its scratch: the others whose codes
+// the split path would hold there, also where the one-pass kernel, which needs
+// none, would run them.
+static bool noalloc_refuses(const RowsArgs& a, bool wide, size_t cap) {
+    return !noalloc_scratch_free(a, wide) && noalloc_need(a, wide) > cap;
 }
 
 static int int8_per_token(const nflow_int8_linear_params* p, int64_t M, const float* A,
@@ -1036,11 +1038,13 @@ static int int8_per_token(const nflow_int8_linear_params* p, int64_t M, const fl
         launch_skinny_i8(a, act_x2, st);
         return finish();
     }
-    // The split form allocates: not where its codes exceed the no-allocation
-    // scratch, nor for a capture that the one-pass kernel can serve.
+    // The split form takes a workspace: not where the no-allocation entry
+    // point's callers rely on the shape using none, nor for a capture that the
+    // one-pass kernel can serve.
     const bool one_pass = use_token_gemm(a);
-    if (!refused && one_pass && !(wide && split_faster(a) && !(fixed && noalloc_need(a, wide) > fixed->cap) &&
-                                  !(a.K <= 512 && !fixed && stream_capturing(st)))) {
+    const bool split = wide && split_faster(a) && !(fixed && noalloc_scratch_free(a, wide)) &&
+                       !(a.K <= 512 && !fixed && stream_capturing(st));
+    if (!refused && one_pass && !split) {
         launch_token_i8(a, act_x2, st);
         return finish();
     }
