@@ -619,7 +619,10 @@ struct Scratch {
     Scratch& operator=(const Scratch&) = delete;
 };
 
-// Whether a graph capture is recording stream st.
+// Whether a graph capture is recording stream st.  A workspace would then be
+// allocated inside the graph (a chain of layers recorded that way took an
+// illegal memory access on its first replay), so layers the one-pass kernel
+// can serve take it, also where the split form is the faster one.
 static bool stream_capturing(hipStream_t st) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
@@ -734,7 +737,7 @@ static int int8_fixed_path(const nflow_int8_linear_params* p, int64_t rows, cons
     RowsArgs g = a;
     g.Aq = nullptr;  // the codes go to the workspace, which is 256-byte aligned
     const bool wide = aligned(A, 16) && use_gemm(g);
-    if (use_token_gemm(a) && !(wide && fixed_split_faster(a))) {
+    if (use_token_gemm(a) && !(wide && fixed_split_faster(a) && !stream_capturing(st))) {
         launch_token_i8_fixed(a, st);
         return check_launch(what);
     }
@@ -1042,8 +1045,7 @@ static int int8_per_token(const nflow_int8_linear_params* p, int64_t M, const fl
     // point's callers rely on the shape using none, nor for a capture that the
     // one-pass kernel can serve.
     const bool one_pass = use_token_gemm(a);
-    const bool split = wide && split_faster(a) && !(fixed && noalloc_scratch_free(a, wide)) &&
-                       !(a.K <= 512 && !fixed && stream_capturing(st));
+    const bool split = wide && split_faster(a) && (fixed ? !noalloc_scratch_free(a, wide) : !stream_capturing(st));
     if (!refused && one_pass && !split) {
         launch_token_i8(a, act_x2, st);
         return finish();
@@ -1302,7 +1304,7 @@ static int fp8_per_token(const nflow_fp8_linear_params* p, int64_t M, const floa
     RowsArgs g = a;
     g.Aq = nullptr;  // the codes go to the workspace, which is 256-byte aligned
     const bool wide = a.K >= 512 && use_gemm(g);
-    if (use_token_gemm(a) && !(wide && fp8_split_faster(a))) {
+    if (use_token_gemm(a) && !(wide && fp8_split_faster(a) && !stream_capturing(st))) {
         launch_token_fp8(a, act_x2, st);
         return finish();
     }

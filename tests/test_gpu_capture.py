@@ -5,12 +5,14 @@ graph (the others).  The recorded nodes are counted before any replay; then
 every replay, with eager work between, must equal the eager call."""
 import ctypes as C
 
+import numpy as np
 import pytest
 import torch
 
 from neuroflow_amd import _lib
 from neuroflow_amd import quant as Q
 from neuroflow_amd import workloads as WL
+from oracle import oracle as O
 from tests.test_gpu_one_pass import _cu, _int8
 
 pytestmark = pytest.mark.gpu
@@ -80,3 +82,45 @@ def test_noalloc_shapes_without_scratch_are_one_kernel(gpu, M, K, N):
     assert _node_types(g) == [KERNEL]
     other = torch.empty_like(want)
     _replays_equal(g, out, want, lambda: call(other))
+
+
+# Shapes that run as quantise + GEMM outside a capture.
+@pytest.mark.parametrize("kind,M,K,N", [("int8", 8192, 512, 1024), ("int8", 4096, 1024, 1024), ("int8", 3000, 960, 300),
+                                        ("fp8", 4096, 1024, 1024), ("fp8", 20000, 512, 2048), ("rows", 8192, 512, 2048),
+                                        ("rows", 4096, 1024, 256), ("batched", 2000, 640, 512)])
+def test_layers_up_to_1024_allocate_nothing_in_a_graph(gpu, kind, M, K, N):
+    """Layers of K <= 1024 record one kernel: no workspace inside the graph.
+    The replays equal the eager one-pass kernel (no_gemm keeps it off the
+    GEMM), and INT8 the eager call as it runs by itself."""
+    L = _lib.lib()
+    if kind == "fp8":
+        qw, sw = O.quantise_weight_fp8(WL.uniform(610, (N, K), -0.125, 0.125))
+        p = Q.Fp8LinearParams(_cu(qw, 0), _cu(sw, 0))
+    else:
+        q, s, zps, sw, b = _int8(N, K, 611)
+        fixed = kind != "int8"
+        p = Q.Int8LinearParams(_cu(q, 0), _cu(s, 0), _cu(zps, 0) if fixed else None, _cu(b, 0), 0.02, 3,
+                               _cu(sw, 0) if fixed else None)
+    fn, args = {"int8": (L.nflow_int8_linear_forward_per_token, (None, 1)),
+                "fp8": (L.nflow_fp8_linear_forward_per_token, (None, 1)),
+                "rows": (L.nflow_int8_linear_forward_rows, ()),
+                "batched": (L.nflow_int8_linear_forward_batched, ())}[kind]
+    ps = p.c_struct()
+    x = torch.from_numpy(WL.normal(614, (M, K)).astype(np.float32)).cuda()
+
+    def call(out):
+        _lib.check(fn(C.byref(ps), M, x.data_ptr(), out.data_ptr(), *args, _stream()), kind)
+
+    eager, want, out = (torch.empty(M, N, device="cuda") for _ in range(3))
+    call(eager)
+    prev = C.c_int(0)
+    _lib.check(L.nflow_debug_set_kernel_path(b"no_gemm", 1, C.byref(prev)), "path")
+    try:
+        call(want)
+    finally:
+        _lib.check(L.nflow_debug_set_kernel_path(b"no_gemm", prev.value, None), "path")
+    if kind != "fp8":
+        assert torch.equal(eager.view(torch.int32), want.view(torch.int32))
+    g = _captured(call, out)
+    assert _node_types(g) == [KERNEL]
+    _replays_equal(g, out, want, lambda: call(eager))
