@@ -1045,7 +1045,10 @@ static int int8_per_token(const nflow_int8_linear_params* p, int64_t M, const fl
     // point's callers rely on the shape using none, nor for a capture that the
     // one-pass kernel can serve.
     const bool one_pass = use_token_gemm(a);
-    const bool split = wide && split_faster(a) && (fixed ? !noalloc_scratch_free(a, wide) : !stream_capturing(st));
+    // On the per-thread default stream a workspace costs an allocation and a
+    // free per call: shapes that need none keep to that.
+    const bool none_taken = (fixed || st == hipStreamPerThread) && noalloc_scratch_free(a, wide);
+    const bool split = wide && split_faster(a) && !none_taken && (fixed || !stream_capturing(st));
     if (!refused && one_pass && !split) {
         launch_token_i8(a, act_x2, st);
         return finish();

@@ -1,4 +1,4 @@
-"""What a layer call records into a graph.  A call whose shape needs no
+"""What a layer call allocates, and what it records into a graph.  A call whose shape needs no
 workspace must stay one kernel; a workspace would be one array shared by
 unordered streams (the no-allocation entry point) or an allocation inside the
 graph (the others).  The recorded nodes are counted before any replay; then
@@ -124,3 +124,36 @@ def test_layers_up_to_1024_allocate_nothing_in_a_graph(gpu, kind, M, K, N):
     g = _captured(call, out)
     assert _node_types(g) == [KERNEL]
     _replays_equal(g, out, want, lambda: call(eager))
+
+
+def _pool_used_high(reset=False):
+    """High-water mark of the device's default pool of stream-ordered allocations."""
+    hip, pool, v = _hip(), C.c_void_p(), C.c_uint64(0)
+    assert hip.hipDeviceGetDefaultMemPool(C.byref(pool), torch.cuda.current_device()) == 0
+    USED_CURRENT, USED_HIGH = 7, 8   # hipMemPoolAttrUsedMemCurrent, hipMemPoolAttrUsedMemHigh
+    if reset:
+        assert hip.hipMemPoolSetAttribute(pool, USED_HIGH, C.byref(v)) == 0
+        assert hip.hipMemPoolGetAttribute(pool, USED_CURRENT, C.byref(v)) == 0
+    else:
+        assert hip.hipMemPoolGetAttribute(pool, USED_HIGH, C.byref(v)) == 0
+    return v.value
+
+
+@pytest.mark.parametrize("M,K,N,allocates", [(8192, 512, 1024, False), (9000, 256, 512, False), (4096, 1024, 256, True)])
+def test_per_thread_stream_keeps_workspace_free_shapes(gpu, M, K, N, allocates):
+    """The per-thread default stream keeps no workspace (a call that takes one
+    allocates and frees it): shapes that need none take none there.  The
+    K = 1024 row shows that the mark moves when a call does allocate."""
+    PER_THREAD = 2   # hipStreamPerThread
+    q, s, _, _, b = _int8(N, K, 620)
+    p = Q.Int8LinearParams(_cu(q, 0), _cu(s, 0), None, _cu(b, 0))
+    ps = p.c_struct()
+    x = torch.from_numpy(WL.normal(623, (M, K))).cuda()
+    want, out = Q.linear_forward_per_token(p, x, "relu"), torch.empty(M, N, device="cuda")
+    torch.cuda.synchronize()
+    before = _pool_used_high(reset=True)
+    _lib.check(_lib.lib().nflow_int8_linear_forward_per_token(C.byref(ps), M, x.data_ptr(), out.data_ptr(), None, 1,
+                                                              PER_THREAD), "per token")
+    torch.cuda.synchronize()
+    assert (_pool_used_high() > before) == allocates
+    assert torch.equal(out.view(torch.int32), want.view(torch.int32))
