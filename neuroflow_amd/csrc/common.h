@@ -360,16 +360,36 @@ __device__ __forceinline__ IntEpi int_epi_consts(int formula, int32_t K, int32_t
     return e;
 }
 
+__device__ __forceinline__ int32_t int_epi_t32(const IntEpi& e, int32_t D, int32_t SA) {
+    return static_cast<int32_t>(static_cast<uint32_t>(D) + static_cast<uint32_t>(e.c0) +
+                                static_cast<uint32_t>(e.c1) * static_cast<uint32_t>(SA));
+}
+
+// zp_A = 0 (c2 = 0: every per-token layer) first, a compare and a conversion:
+// testing for overflow before it cost those layers 10 to 20% (row-tile kernel
+// on codes, 20000 x 4 -> 1000, 72 -> 84 us).  Then the 64-bit sum as a 32-bit
+// one wherever that holds it (the conversion to float rounds the same
+// integer): the 64-bit conversion costs several times the rest of the epilogue.
 __device__ __forceinline__ float int_epi_value(const IntEpi& e, int32_t D, int32_t SA) {
-    const uint32_t t32 = static_cast<uint32_t>(D) + static_cast<uint32_t>(e.c0) +
-                         static_cast<uint32_t>(e.c1) * static_cast<uint32_t>(SA);
-    // The 64-bit sum as a 32-bit one wherever that holds it (the conversion
-    // to float then rounds the same integer): the 64-bit conversion costs
-    // several times the rest of the epilogue.
-    const int32_t t = static_cast<int32_t>(t32), c2 = static_cast<int32_t>(e.c2);
+    const int32_t t = int_epi_t32(e, D, SA);
+    if (e.c2 == 0) return static_cast<float>(t);
+    const int32_t c2 = static_cast<int32_t>(e.c2);
     int32_t u;
     if (c2 == e.c2 && !__builtin_add_overflow(t, c2, &u)) return static_cast<float>(u);
     return static_cast<float>(static_cast<int64_t>(t) + e.c2);
+}
+
+// Whether the whole integer epilogue of a column stays inside 32 bits for any
+// codes (|D| <= 2^14 K, |SA| <= 2^7 K), with c1 in 24: then t is
+// D + (c0 + c2) + mul24(c1, SA), every step exact.  Zero points of 8 bits
+// always pass for K <= 1024.
+__device__ __forceinline__ bool int_epi_small(const IntEpi& e, int32_t K) {
+    const double c0 = e.c0, c1 = e.c1, c2 = static_cast<double>(e.c2), k = K;
+    return __builtin_fabs(c1) < 0x1p23 &&
+           __builtin_fabs(c0) + __builtin_fabs(c2) + k * (0x1p14 + 0x1p7 * __builtin_fabs(c1)) < 0x1p31;
+}
+__device__ __forceinline__ float int_epi_value_small(int32_t c02, int32_t c1, int32_t D, int32_t SA) {
+    return static_cast<float>(D + c02 + __mul24(c1, SA));
 }
 
 // The FNO layer's INT8 fake-quant of x2 (fno.cpp:626-646 per-position,

@@ -51,7 +51,7 @@
 // the K loop (one coalesced load each, whose latency the K loop covers),
 // forms the INT8 epilogue constants from the weight bytes summed during the K
 // loop (as in the row-tile kernels) and files everything in the wave's LDS
-// tables, which the epilogue reads as float4 / IntEpi per lane.  Loading them
+// tables, which the epilogue reads as 16-byte vectors per lane.  Loading them
 // per output lane after the K loop instead puts a chain of dependent global
 // loads -- each also waiting for the previous chunk's stores -- between
 // every product and its stores.
@@ -244,7 +244,9 @@ __device__ __forceinline__ void token_tile_gemm(const RowsArgs& a, const uint8_t
     const int r = lane & 15, g = lane >> 4;
     const int64_t M = a.M;
     const int N = a.N;
-    IntEpi* etab = reinterpret_cast<IntEpi*>(ctab);                     // the wave's columns' INT8 constants
+    int32_t* c0tab = reinterpret_cast<int32_t*>(ctab);                  // the wave's columns' INT8 constants
+    int32_t* c1tab = c0tab + 64;
+    int64_t* c2tab = reinterpret_cast<int64_t*>(c1tab + 64);
     float* swtab = reinterpret_cast<float*>(ctab + 64 * sizeof(IntEpi));  // weight scales
     float* btab = swtab + 64;                                             // biases
     const int64_t w_total = static_cast<int64_t>(N) * K;
@@ -343,7 +345,7 @@ __device__ __forceinline__ void token_tile_gemm(const RowsArgs& a, const uint8_t
         }
         // Weight byte sums of column 16 ct + r reduced over the lane groups;
         // lane (r, g) = column 16 g + r takes tile ct = g.
-        bool trivial = true;
+        bool trivial = true, small = true;
         if constexpr (SUMS) {
             int32_t wfull = 0, wd = 0;
 #pragma unroll
@@ -359,9 +361,15 @@ __device__ __forceinline__ void token_tile_gemm(const RowsArgs& a, const uint8_t
             const int32_t my_zp = a.zpW ? my_zp0 : 0;
             const IntEpi mine = int_epi_consts(a.formula, K, a.zp_A, my_zp, a.sumW ? my_sg0 : 0,
                                                a.sumW != nullptr, wfull, wd);
-            // Wave-uniform: all the columns' constants zero, the result is (float)D.
+            // Wave-uniform: all the columns' constants zero, the result is
+            // (float)D; or no column's sum can leave 32 bits.
             trivial = !__any((mine.c0 != 0) | (mine.c1 != 0) | (mine.c2 != 0));
-            if (!trivial && lane < S::WCOLS) etab[lane] = mine;
+            small = !__any(!int_epi_small(mine, K));
+            if (!trivial && lane < S::WCOLS) {
+                c0tab[lane] = small ? mine.c0 + static_cast<int32_t>(mine.c2) : mine.c0;
+                c1tab[lane] = mine.c1;
+                c2tab[lane] = mine.c2;
+            }
         }
         if (CT == 4 || lane < S::WCOLS) {
             swtab[lane] = my_sw;
@@ -379,9 +387,17 @@ __device__ __forceinline__ void token_tile_gemm(const RowsArgs& a, const uint8_t
 #pragma unroll
                     for (int v = 0; v < 4; ++v) t[v] = static_cast<float>(acc[rt][ct][v]);
                 } else {
+                    const v4i e0 = *reinterpret_cast<const v4i*>(c0tab + c0), e1 = *reinterpret_cast<const v4i*>(c1tab + c0);
+                    if (small) {
 #pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        t[v] = int_epi_value(etab[c0 + v], static_cast<int32_t>(acc[rt][ct][v]), sarow[rt]);
+                        for (int v = 0; v < 4; ++v)
+                            t[v] = int_epi_value_small(e0[v], e1[v], static_cast<int32_t>(acc[rt][ct][v]), sarow[rt]);
+                    } else {
+#pragma unroll
+                        for (int v = 0; v < 4; ++v)
+                            t[v] = int_epi_value(IntEpi{e0[v], e1[v], c2tab[c0 + v]}, static_cast<int32_t>(acc[rt][ct][v]),
+                                                 sarow[rt]);
+                    }
                 }
                 const v4f sw4 = *reinterpret_cast<const v4f*>(swtab + c0);
                 const v4f b4 = *reinterpret_cast<const v4f*>(btab + c0);

@@ -183,3 +183,25 @@ def test_square_layer_in_place(gpu, M, K, fmt):
             assert torch.allclose(y, out, rtol=1e-5, atol=1e-5)
         else:
             assert torch.equal(y.view(torch.int32), out.view(torch.int32))
+
+
+# Zero points within 8 bits (the 32-bit epilogue), at the edge of 24 bits and
+# beyond, where its products and the 64-bit term need the general form.
+@pytest.mark.parametrize("zp_w,zp_a", [(127, -128), (1 << 21, 3), ((1 << 22) + 1, 3), (1 << 24, 100000), (1 << 30, 0)])
+@pytest.mark.parametrize("M,K,N", [(70, 100, 65), (33, 512, 128), (20, 1000, 36), (65, 60, 260)])
+def test_zero_point_range(gpu, tile_rows, zp_w, zp_a, M, K, N):
+    W = WL.uniform(890, (N, K), -0.125, 0.125)
+    s = O.per_channel_scales(W, 127.0)
+    zps = WL.uniform(891, (N,), -zp_w, zp_w).astype(np.int32)
+    zps[:2] = zp_w, -zp_w
+    q, sw = O.quantise_weight_2d(W, s, zps)
+    b = WL.uniform(892, (N,), -0.1, 0.1)
+    A = WL.normal(893, (M, K))
+    p = Q.Int8LinearParams(_cu(q, 0), _cu(s, 0), _cu(zps, 0), _cu(b, 0), 0.02, zp_a, _cu(sw, 0))
+    want, _ = O.layer_per_token_i8(A, q, s, zps, b, sw, 0)
+    got = Q.linear_forward_per_token(p, _cu(A, 0), "none").cpu().numpy()
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    for fn, ref in ((Q.linear_forward_batched, O.linear_forward_batched), (Q.linear_forward, O.linear_forward_rows)):
+        rc, want = ref(A, q, s, zps, b, 0.02, zp_a, sw)
+        assert rc == 0
+        assert np.array_equal(fn(p, _cu(A, 0)).cpu().numpy().view(np.uint32), want.view(np.uint32))
