@@ -40,14 +40,19 @@ static void launch_token_rag(const RowsArgs& a, int act, hipStream_t st) {
     else if constexpr (RT == 1) launch_token_act<16, FMT, CT, RT, true>(a, act, st);
 }
 
+template <int FMT, int CT>
+static void launch_token_whole(const RowsArgs& a, int act, hipStream_t st) {
+    if (a.K == 128) launch_token_act<2, FMT, CT, 4, false>(a, act, st);
+    else if (a.K == 256) launch_token_act<4, FMT, CT, 4, false>(a, act, st);
+    else launch_token_act<8, FMT, CT, 4, false>(a, act, st);
+}
+
 template <int FMT>
 static void launch_token_fmt(const RowsArgs& a, int act, hipStream_t st) {
     if (token_small_tiles(a)) return launch_token_rag<FMT, 2, 1>(a, act, st);
-    if (a.N <= 128) return launch_token_rag<FMT, 2, 4>(a, act, st);
-    if (!token_whole(a)) return launch_token_rag<FMT, 4, 4>(a, act, st);
-    if (a.K == 128) launch_token_act<2, FMT, 4, 4, false>(a, act, st);
-    else if (a.K == 256) launch_token_act<4, FMT, 4, 4, false>(a, act, st);
-    else launch_token_act<8, FMT, 4, 4, false>(a, act, st);
+    if (!token_whole(a)) return a.N <= 128 ? launch_token_rag<FMT, 2, 4>(a, act, st) : launch_token_rag<FMT, 4, 4>(a, act, st);
+    if (a.N <= 128) launch_token_whole<FMT, 2>(a, act, st);
+    else launch_token_whole<FMT, 4>(a, act, st);
 }
 
 }  // namespace nfq

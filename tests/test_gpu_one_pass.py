@@ -205,3 +205,32 @@ def test_zero_point_range(gpu, tile_rows, zp_w, zp_a, M, K, N):
         rc, want = ref(A, q, s, zps, b, 0.02, zp_a, sw)
         assert rc == 0
         assert np.array_equal(fn(p, _cu(A, 0)).cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("M", [1, 63, 64, 65, 200, 6000])
+@pytest.mark.parametrize("K,N", [(128, 64), (256, 128), (512, 64), (512, 128), (256, 192)])
+def test_whole_shapes(gpu, tile_rows, M, K, N):
+    """Whole K blocks and column strips at aligned buffers, the narrow (N <= 128)
+    and the wide form, in the three formats."""
+    q, s, zps, sw, b = _int8(N, K, 895)
+    A = WL.normal(898, (M, K))
+    rows = _rows(M)
+    p = Q.Int8LinearParams(_cu(q, 0), _cu(s, 0), _cu(zps, 0), _cu(b, 0), 0.02, 5, _cu(sw, 0))
+    buf, out = _guarded(M, N, 0)
+    y = Q.linear_forward_per_token(p, _cu(A, 0), "relu", out=out).cpu().numpy()[rows]
+    want, _ = O.layer_per_token_i8(A[rows], q, s, zps, b, sw, 1)
+    assert np.array_equal(y.view(np.uint32), want.view(np.uint32))
+    assert _guards_kept(buf, M, N, 0)
+    y = Q.linear_forward_batched(p, _cu(A, 0)).cpu().numpy()[rows]
+    rc, want = O.linear_forward_batched(A[rows], q, s, zps, b, 0.02, 5, sw)
+    assert rc == 0 and np.array_equal(y.view(np.uint32), want.view(np.uint32))
+    qw, s8 = O.quantise_weight_fp8(WL.uniform(899, (N, K), -0.125, 0.125))
+    buf, out = _guarded(M, N, 0)
+    y = Q.fp8_linear_forward_per_token(Q.Fp8LinearParams(_cu(qw, 0), _cu(s8, 0), _cu(b, 0)), _cu(A, 0), "none", out=out)
+    assert _guards_kept(buf, M, N, 0)
+    qa, sa = O.quantise_per_token_fp8(A[rows])
+    want = O.layer_fp8_exact(qa, sa, qw, s8, b, 0)
+    terms = (np.abs(O.e4m3_decode(qa)) * sa[:, None]).astype(np.float64) @ \
+        (np.abs(O.e4m3_decode(qw)) * s8[:, None]).astype(np.float64).T
+    bound = (K + 3) * 2.0 ** -24 * (terms + np.abs(b)[None, :]) + 1e-38
+    assert np.all(np.abs(y.cpu().numpy()[rows].astype(np.float64) - want) <= bound)
