@@ -365,18 +365,31 @@ __device__ __forceinline__ int32_t int_epi_t32(const IntEpi& e, int32_t D, int32
                                 static_cast<uint32_t>(e.c1) * static_cast<uint32_t>(SA));
 }
 
-// zp_A = 0 (c2 = 0: every per-token layer) first, a compare and a conversion:
-// testing for overflow before it cost those layers 10 to 20% (row-tile kernel
-// on codes, 20000 x 4 -> 1000, 72 -> 84 us).  Then the 64-bit sum as a 32-bit
-// one wherever that holds it (the conversion to float rounds the same
-// integer): the 64-bit conversion costs several times the rest of the epilogue.
-__device__ __forceinline__ float int_epi_value(const IntEpi& e, int32_t D, int32_t SA) {
-    const int32_t t = int_epi_t32(e, D, SA);
-    if (e.c2 == 0) return static_cast<float>(t);
-    const int32_t c2 = static_cast<int32_t>(e.c2);
+// Per-token layers: zp_A = 0, so c2 = 0.
+__device__ __forceinline__ float int_epi_value_token(const IntEpi& e, int32_t D, int32_t SA) {
+    return static_cast<float>(int_epi_t32(e, D, SA));
+}
+
+// Fixed-scale layers, whose c2 is rarely 0: the 64-bit sum as a 32-bit one
+// wherever that holds it (the conversion to float then rounds the same
+// integer), as the 64-bit conversion costs several times the rest of the
+// epilogue.
+__device__ __forceinline__ float int_epi_value_fixed(const IntEpi& e, int32_t D, int32_t SA) {
+    const int32_t t = int_epi_t32(e, D, SA), c2 = static_cast<int32_t>(e.c2);
     int32_t u;
     if (c2 == e.c2 && !__builtin_add_overflow(t, c2, &u)) return static_cast<float>(u);
     return static_cast<float>(static_cast<int64_t>(t) + e.c2);
+}
+
+// Kernels that serve both: testing for overflow where c2 = 0 cost per-token
+// layers 10 to 20% (row-tile kernel on codes, 20000 x 4 -> 1000, 72 -> 84 us),
+// testing for c2 = 0 fixed-scale ones 0.2 to 0.5 us in small launches.
+template <bool FIXED>
+__device__ __forceinline__ float int_epi_value_of(const IntEpi& e, int32_t D, int32_t SA) {
+    return FIXED ? int_epi_value_fixed(e, D, SA) : int_epi_value_token(e, D, SA);
+}
+__device__ __forceinline__ float int_epi_value(const IntEpi& e, int32_t D, int32_t SA) {
+    return e.c2 == 0 ? int_epi_value_token(e, D, SA) : int_epi_value_fixed(e, D, SA);
 }
 
 // Whether the whole integer epilogue of a column stays inside 32 bits for any

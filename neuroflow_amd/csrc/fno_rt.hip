@@ -1396,7 +1396,7 @@ __global__ __launch_bounds__(256) void k_layer_tail(LayerTailArgs la) {
             for (int v = 0; v < 4; ++v) {
                 const int ch = 32 * chh + 16 * ct + 4 * g + v;
                 float t;
-                if constexpr (INT_EPI) t = int_epi_value(cepi[ch], acc[v], SA);
+                if constexpr (INT_EPI) t = int_epi_value_fixed(cepi[ch], acc[v], SA);
                 else t = static_cast<float>(acc[v]);
                 const float x2 = dequant_bias(csw[ch], la.sA, t, cbias[ch]);
                 float ps = 0.0f, pz = 0.0f;

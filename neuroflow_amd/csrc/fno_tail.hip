@@ -197,7 +197,7 @@ __global__ __launch_bounds__(256) void k_layer_tail_w(LayerTailArgs la, int int_
             if (int_epi) {
 #pragma unroll
                 for (int k = 0; k < KQ; ++k) SA = sum_bytes_i8(cr[k], SA);
-                tv = int_epi_value(epi, D, SA);
+                tv = int_epi_value_fixed(epi, D, SA);
             } else {
                 tv = static_cast<float>(D);
             }

@@ -503,7 +503,7 @@ __global__ __launch_bounds__(64 * WPB, WPB == 4 ? 3 : 1) void k_rows64(RowsArgs 
                 for (int v = 0; v < 4; ++v) t[v] = static_cast<float>(acc_i[v]);
             } else {
 #pragma unroll
-                for (int v = 0; v < 4; ++v) t[v] = int_epi_value(lds_e[16 * nt + 4 * g + v], acc_i[v], SA);
+                for (int v = 0; v < 4; ++v) t[v] = int_epi_value_of<FIXED>(lds_e[16 * nt + 4 * g + v], acc_i[v], SA);
             }
             const v4f sw = lds_sw[4 * nt + g];
             const v4f bb = lds_b[4 * nt + g];

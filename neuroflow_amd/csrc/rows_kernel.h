@@ -245,7 +245,7 @@ __device__ __forceinline__ void gather_consts(const IntEpi& mine, int g, IntEpi 
     }
 }
 
-template <bool FP8, int ACT, int OUT>
+template <bool FP8, int ACT, int OUT, bool FIXED>
 __device__ __forceinline__ void store_tile(const RowsArgs& a, int64_t row, int n0, int g,
                                            const v4i& acc_i, const v4f& acc_f, v4f sw, v4f bias,
                                            bool trivial, const IntEpi* e, float srow,
@@ -271,7 +271,7 @@ __device__ __forceinline__ void store_tile(const RowsArgs& a, int64_t row, int n
             for (int v = 0; v < 4; ++v) t[v] = static_cast<float>(acc_i[v]);
         } else {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) t[v] = int_epi_value(e[v], acc_i[v], SA);
+            for (int v = 0; v < 4; ++v) t[v] = int_epi_value_of<FIXED>(e[v], acc_i[v], SA);
         }
         v4f y;
 #pragma unroll
@@ -528,7 +528,7 @@ __global__ __launch_bounds__(256, rows_min_waves(KB, FP8)) void k_rows(RowsArgs 
                         for (int v = 0; v < 4; ++v) e[v] = lds_e[nt * 16 + 4 * g + v];
                     }
                 }
-                store_tile<FP8, ACT, OUT>(a, row, nt * 16, g, acc_i, acc_f, lds_sw[nt * 4 + g],
+                store_tile<FP8, ACT, OUT, IN == IN_F32_FIXED>(a, row, nt * 16, g, acc_i, acc_f, lds_sw[nt * 4 + g],
                                           lds_b[nt * 4 + g], triv[nt], e, srow, SA);
             }
         } else {
@@ -557,7 +557,7 @@ __global__ __launch_bounds__(256, rows_min_waves(KB, FP8)) void k_rows(RowsArgs 
                     if constexpr (INT_EPI) {
                         if (!cc.trivial) gather_consts(mine, g, e);
                     }
-                    store_tile<FP8, ACT, OUT>(a, row, nc, g, acc_i, acc_f, cc.sw, cc.b, cc.trivial, e,
+                    store_tile<FP8, ACT, OUT, IN == IN_F32_FIXED>(a, row, nc, g, acc_i, acc_f, cc.sw, cc.b, cc.trivial, e,
                                               srow, SA);
                 }
             }

@@ -170,7 +170,7 @@ __global__ __launch_bounds__(64 * NW) void k_skinny(RowsArgs a) {
             }
             const IntEpi e = int_epi_consts(a.formula, K, a.zp_A, a.zpW ? a.zpW[col] : 0, a.sumW ? a.sumW[col] : 0,
                                             a.sumW != nullptr, Sf, Sd);
-            tv = int_epi_value(e, D, SA);
+            tv = int_epi_value_of<FMT == TG_I8_FIXED>(e, D, SA);
         }
         const float srow = FMT == TG_I8_FIXED ? a.scale_A : scale_s[rr];
         const float y = activate<ACT>(dequant_bias(a.sW[col], srow, tv, a.bias ? a.bias[col] : 0.0f));

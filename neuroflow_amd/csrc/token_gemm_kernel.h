@@ -397,8 +397,8 @@ __device__ __forceinline__ void token_tile_gemm(const RowsArgs& a, const uint8_t
                     } else {
 #pragma unroll
                         for (int v = 0; v < 4; ++v)
-                            t[v] = int_epi_value(IntEpi{e0[v], e1[v], c2tab[c0 + v]}, static_cast<int32_t>(acc[rt][ct][v]),
-                                                 sarow[rt]);
+                            t[v] = int_epi_value_of<FMT == TG_I8_FIXED>(IntEpi{e0[v], e1[v], c2tab[c0 + v]},
+                                                                        static_cast<int32_t>(acc[rt][ct][v]), sarow[rt]);
                     }
                 }
                 const v4f sw4 = *reinterpret_cast<const v4f*>(swtab + c0);
