@@ -33,35 +33,43 @@ namespace nfq {
 
 // The elementwise kernels are bound by HBM.  A thread takes kElemQuads groups
 // of four elements, 256 groups apart: 16-byte and 4-byte accesses of whole
-// wave-contiguous segments, all of a thread's loads in flight at once; the
-// last n % 4 elements, and buffers the accesses do not fit (vec = 0), go one
-// by one.  (One element per thread with byte accesses ran E4M3 encode 23.0
-// and decode 18.6 us at 16 Mi elements, 84 MB each; this form 16.4 and 12.8.)
+// wave-contiguous segments, all of a thread's loads in flight at once; one
+// group (per = 1) where four would leave the CUs under two blocks; the last
+// n % 4 elements, and buffers the accesses do not fit (per = 0), go one by one,
+// an element per thread.  (That form alone ran E4M3 encode 23.0 and decode
+// 18.6 us at 16 Mi elements, 84 MB each; this one 16.4 and 12.8.  With the
+// four-group grid throughout, decode of 1 Mi ran 3.6 us for 3.3, and an
+// unaligned encode of 1 Mi 6.3.)
 constexpr int kElemQuads = 4;
 
-// f4(quad index) over whole quads, f1(element index) over the rest.
+// f4(first quad, end of the block's quads) over whole quads, f1(element index)
+// over the rest.
 template <typename F4, typename F1>
-__device__ __forceinline__ void each_quad(int64_t n, int vec, F4 f4, F1 f1) {
-    const int64_t nq = vec ? n / 4 : 0;
-    for (int64_t b = static_cast<int64_t>(blockIdx.x) * (256 * kElemQuads); b < nq;
-         b += static_cast<int64_t>(gridDim.x) * (256 * kElemQuads))
-        f4(b + threadIdx.x, nq);
+__device__ __forceinline__ void each_quad(int64_t n, int per, F4 f4, F1 f1) {
+    const int64_t nq = per ? n / 4 : 0, span = 256 * per;
+    for (int64_t b = static_cast<int64_t>(blockIdx.x) * span; b < nq; b += static_cast<int64_t>(gridDim.x) * span)
+        f4(b + threadIdx.x, b + span < nq ? b + span : nq);
     for (int64_t i = 4 * nq + static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < n;
          i += static_cast<int64_t>(gridDim.x) * 256)
         f1(i);
 }
 
-// The launch of an elementwise kernel over n elements.
-static dim3 elem_grid(int64_t n) { return dim3(grid_for((n + 3) / 4, 256 * kElemQuads, 16)); }
+// The launch of an elementwise kernel over n elements: groups per thread, grid.
+static int elem_per(int64_t n, bool aligned_buffers) {
+    return !aligned_buffers ? 0 : n / 4 <= static_cast<int64_t>(num_cus()) * 2 * 256 * kElemQuads ? 1 : kElemQuads;
+}
+static dim3 elem_grid(int64_t n, int per) {
+    return dim3(per ? grid_for((n + 3) / 4, 256 * per, 16) : grid_for(n, 256, 16));
+}
 
 // QuantiseActivation, int8_gemm.cpp:507-520.
 __global__ __launch_bounds__(256) void k_quantise_fixed(const float* __restrict__ A,
                                                         int8_t* __restrict__ Aq, int64_t n,
-                                                        float s, int32_t zp, int vec) {
+                                                        float s, int32_t zp, int per) {
     const float inv = 1.0f / s;
     const bool fast = s >= 0x1p-120f && s <= 0x1p120f;   // the reciprocal path's range
     each_quad(
-        n, vec,
+        n, per,
         [&](int64_t q0, int64_t nq) {
             v4f x[kElemQuads];
 #pragma unroll
@@ -220,9 +228,9 @@ __device__ __forceinline__ uint32_t e4m3_encode4(v4f x) {
 }
 
 __global__ __launch_bounds__(256) void k_e4m3_encode(const float* __restrict__ in,
-                                                     uint8_t* __restrict__ out, int64_t n, int vec) {
+                                                     uint8_t* __restrict__ out, int64_t n, int per) {
     each_quad(
-        n, vec,
+        n, per,
         [&](int64_t q0, int64_t nq) {
             v4f x[kElemQuads];
 #pragma unroll
@@ -236,9 +244,9 @@ __global__ __launch_bounds__(256) void k_e4m3_encode(const float* __restrict__ i
 }
 
 __global__ __launch_bounds__(256) void k_e4m3_decode(const uint8_t* __restrict__ in,
-                                                     float* __restrict__ out, int64_t n, int vec) {
+                                                     float* __restrict__ out, int64_t n, int per) {
     each_quad(
-        n, vec,
+        n, per,
         [&](int64_t q0, int64_t nq) {
             uint32_t b[kElemQuads];
 #pragma unroll
@@ -258,7 +266,7 @@ __global__ __launch_bounds__(256) void k_e4m3_decode(const uint8_t* __restrict__
 
 // fp8_e4m3_per_tensor_fake_quant, fp8_e4m3.h:312-334 (in == out allowed).
 __global__ __launch_bounds__(256) void k_fp8_fake_quant(const float* in, float scale, float* out,
-                                                        int64_t n, int vec) {
+                                                        int64_t n, int per) {
     const float inv = (scale == 0.0f) ? 1.0f : (1.0f / scale);
     // The byte's value; the byte of a NaN decodes to the positive quiet NaN.
     auto value = [&](float x) {
@@ -266,7 +274,7 @@ __global__ __launch_bounds__(256) void k_fp8_fake_quant(const float* in, float s
         return (__builtin_isnan(xs) ? __uint_as_float(0x7FC00000u) : fp8_value_of(xs)) * scale;
     };
     each_quad(
-        n, vec,
+        n, per,
         [&](int64_t q0, int64_t nq) {
             v4f x[kElemQuads];
 #pragma unroll
@@ -776,8 +784,9 @@ static int int8_fixed_path(const nflow_int8_linear_params* p, int64_t rows, cons
     Scratch ws(static_cast<size_t>(rows) * a.K, st);
     if (ws.err != hipSuccess) return set_error(NFLOW_INTERNAL, std::string(what) + ": workspace allocation failed");
     const int64_t n = rows * a.K;
-    hipLaunchKernelGGL(k_quantise_fixed, elem_grid(n), dim3(256), 0, st, A, static_cast<int8_t*>(ws.p), n,
-                       p->scale_A, p->zp_A, aligned(A, 16));
+    const int per = elem_per(n, aligned(A, 16));
+    hipLaunchKernelGGL(k_quantise_fixed, elem_grid(n, per), dim3(256), 0, st, A, static_cast<int8_t*>(ws.p), n,
+                       p->scale_A, p->zp_A, per);
     a.Aq = static_cast<const uint8_t*>(ws.p);
     a.scale_in = nullptr;
     launch_generic<false, OUT_EPI>(a, ACT_NONE, st);
@@ -831,8 +840,9 @@ int nflow_int8_quantise_activation(const float* A, int8_t* A_q, int64_t bsz, int
     if (!A || !A_q) return NFLOW_OK;   // the reference returns silently (int8_gemm.cpp:511)
     const int64_t n = bsz * static_cast<int64_t>(in_features);
     if (n <= 0) return NFLOW_OK;
-    hipLaunchKernelGGL(k_quantise_fixed, elem_grid(n), dim3(256), 0, as_stream(stream), A, A_q, n, scale_A, zp_A,
-                       aligned(A, 16) && aligned(A_q, 4));
+    const int per = elem_per(n, aligned(A, 16) && aligned(A_q, 4));
+    hipLaunchKernelGGL(k_quantise_fixed, elem_grid(n, per), dim3(256), 0, as_stream(stream), A, A_q, n, scale_A, zp_A,
+                       per);
     return check_launch("QuantiseActivation");
 }
 
@@ -1224,8 +1234,8 @@ int nflow_fp8_e4m3_to_bits(const float* in, uint8_t* out, int64_t n, void* strea
     clear_error();
     if (!in || !out) return set_error(NFLOW_INVALID_ARG, "fp8_e4m3_to_bits: null pointer");
     if (n <= 0) return NFLOW_OK;
-    hipLaunchKernelGGL(k_e4m3_encode, elem_grid(n), dim3(256), 0, as_stream(stream), in, out, n,
-                       aligned(in, 16) && aligned(out, 4));
+    const int per = elem_per(n, aligned(in, 16) && aligned(out, 4));
+    hipLaunchKernelGGL(k_e4m3_encode, elem_grid(n, per), dim3(256), 0, as_stream(stream), in, out, n, per);
     return check_launch("fp8_e4m3_to_bits");
 }
 
@@ -1233,8 +1243,8 @@ int nflow_fp8_e4m3_from_bits(const uint8_t* in, float* out, int64_t n, void* str
     clear_error();
     if (!in || !out) return set_error(NFLOW_INVALID_ARG, "fp8_e4m3_from_bits: null pointer");
     if (n <= 0) return NFLOW_OK;
-    hipLaunchKernelGGL(k_e4m3_decode, elem_grid(n), dim3(256), 0, as_stream(stream), in, out, n,
-                       aligned(in, 4) && aligned(out, 16));
+    const int per = elem_per(n, aligned(in, 4) && aligned(out, 16));
+    hipLaunchKernelGGL(k_e4m3_decode, elem_grid(n, per), dim3(256), 0, as_stream(stream), in, out, n, per);
     return check_launch("fp8_e4m3_from_bits");
 }
 
@@ -1242,8 +1252,8 @@ int nflow_fp8_e4m3_fake_quant(const float* in, float scale, float* out, int64_t 
     clear_error();
     if (!in || !out) return set_error(NFLOW_INVALID_ARG, "fp8_e4m3_fake_quant: null pointer");
     if (n <= 0) return NFLOW_OK;
-    hipLaunchKernelGGL(k_fp8_fake_quant, elem_grid(n), dim3(256), 0, as_stream(stream), in, scale, out, n,
-                       aligned(in, 16) && aligned(out, 16));
+    const int per = elem_per(n, aligned(in, 16) && aligned(out, 16));
+    hipLaunchKernelGGL(k_fp8_fake_quant, elem_grid(n, per), dim3(256), 0, as_stream(stream), in, scale, out, n, per);
     return check_launch("fp8_e4m3_fake_quant");
 }
 

@@ -66,3 +66,21 @@ def test_quantise_activation(gpu, n, off, scale, zp):
         x[40:80] = (np.arange(40) - 20 + 0.5) * 0.25      # ties at 0.25
     q = Q.quantise_activation(_dev(x, off).view(1, n), scale, zp)
     assert np.array_equal(q.cpu().numpy().reshape(-1), O.quantise_activation(x.reshape(1, n), scale, zp).reshape(-1))
+
+
+# From 2^21 elements a thread takes four groups instead of one: the line, a
+# ragged end, and several passes of the grid.
+@pytest.mark.parametrize("n", [(1 << 21) - 4, 1 << 21, (1 << 21) + 4, 2_500_003, 17_000_001])
+def test_large_tensors(gpu, n):
+    L = _lib.lib()
+    g = torch.Generator(device="cuda").manual_seed(n)
+    t = torch.randn(n, device="cuda", generator=g) * 3.0
+    x = t.cpu().numpy()
+    bits = _call(L.nflow_fp8_e4m3_to_bits, n, t, torch.uint8, 0)
+    assert np.array_equal(bits, O.e4m3_encode(x))
+    vals = _call(L.nflow_fp8_e4m3_from_bits, n, _dev(bits, 0), torch.float32, 0)
+    assert np.array_equal(vals.view(np.uint32), O.e4m3_decode(bits).view(np.uint32))
+    fq = _call(L.nflow_fp8_e4m3_fake_quant, n, t, torch.float32, 0, 0.75)
+    assert np.array_equal(fq.view(np.uint32), O.fp8_fake_quant(x, 0.75).view(np.uint32))
+    q = Q.quantise_activation(t.view(1, n), 0.02, 5)
+    assert np.array_equal(q.cpu().numpy().reshape(-1), O.quantise_activation(x.reshape(1, n), 0.02, 5).reshape(-1))
