@@ -79,16 +79,14 @@ inline bool in_place(const RowsArgs& a) {
     return x && y && x < y + 4 * a.M * a.N && y < x + 4 * a.M * a.K;
 }
 
-// Row-tile kernel eligibility for the given input mode.  On fp32 input it
-// serves K, N <= 64, its weights in registers for the whole launch; the
-// one-pass kernel takes the others (with two K blocks, 100000 x 128 -> 64, the
-// row-tile form ran 42.7 us, the one-pass kernel 28).
+// Row-tile kernel eligibility for the given input mode (on fp32 input it is
+// taken where use_rows says).
 inline bool rows_ok(const RowsArgs& a, int in_mode) {
     if (a.K % 4 != 0 || a.N % 4 != 0) return false;
     if (in_mode == IN_CODES) {
         if (a.K > 1024 || !aligned(a.Aq, 4)) return false;
     } else {
-        if (a.N > 64 || a.K > 64 || !aligned(a.A, 16)) return false;
+        if (a.K > 128 || !aligned(a.A, 16)) return false;
     }
     return aligned(a.W, 4) && aligned(a.C, 16);
 }

@@ -19,13 +19,14 @@ static void launch_rows_k(const RowsArgs& a, hipStream_t st) {
 
 template <int KB, bool FP8, int IN, int OUT, int ACT, bool KFULL>
 static void launch_rows_h(const RowsArgs& a, hipStream_t st) {
-    if constexpr (rows_hoist_fits(KB, FP8)) {
-        if (IN != IN_CODES || a.N <= 64) {
+    // fp32 input at two K blocks: weights per tile (held, they spill).
+    if constexpr (rows_hoist_fits(KB, FP8) && (IN == IN_CODES || KB == 1)) {
+        if (a.N <= 64) {
             launch_rows_k<KB, FP8, IN, OUT, ACT, true, KFULL>(a, st);
             return;
         }
     }
-    if constexpr (IN == IN_CODES) launch_rows_k<KB, FP8, IN, OUT, ACT, false, KFULL>(a, st);
+    launch_rows_k<KB, FP8, IN, OUT, ACT, false, KFULL>(a, st);
 }
 
 template <int KB, bool FP8, int IN, int OUT, int ACT>
@@ -40,7 +41,8 @@ template <bool FP8, int IN, int OUT, int ACT>
 static void launch_rows_act(const RowsArgs& a, hipStream_t st) {
     const int kb = (a.K + 63) / 64;
     if constexpr (IN != IN_CODES) {
-        launch_rows_kb<1, FP8, IN, OUT, ACT>(a, st);   // K <= 64 (rows_ok)
+        if (kb <= 1) launch_rows_kb<1, FP8, IN, OUT, ACT>(a, st);
+        else launch_rows_kb<2, FP8, IN, OUT, ACT>(a, st);   // K <= 128 (rows_ok)
     } else {
         if (kb <= 1) launch_rows_kb<1, FP8, IN, OUT, ACT>(a, st);
         else if (kb <= 2) launch_rows_kb<2, FP8, IN, OUT, ACT>(a, st);

@@ -33,8 +33,10 @@ static void launch_token_act(const RowsArgs& a, int act, hipStream_t st) {
 
 template <int FMT, int CT, int RT>
 static void launch_token_rag(const RowsArgs& a, int act, hipStream_t st) {
-    if (a.K <= 64) launch_token_act<1, FMT, CT, RT, true>(a, act, st);
-    else if (a.K <= 128) launch_token_act<2, FMT, CT, RT, true>(a, act, st);
+    if constexpr (CT == 2) {
+        if (a.K <= 64) return launch_token_act<1, FMT, CT, RT, true>(a, act, st);
+    }
+    if (a.K <= 128) launch_token_act<2, FMT, CT, RT, true>(a, act, st);
     else if (a.K <= 256) launch_token_act<4, FMT, CT, RT, true>(a, act, st);
     else if (RT == 4 || a.K <= 512) launch_token_act<8, FMT, CT, RT, true>(a, act, st);
     else if constexpr (RT == 1) launch_token_act<16, FMT, CT, RT, true>(a, act, st);
@@ -47,11 +49,16 @@ static void launch_token_whole(const RowsArgs& a, int act, hipStream_t st) {
     else launch_token_act<8, FMT, CT, 4, false>(a, act, st);
 }
 
+// 64-row tiles: 32 columns per wave for N <= 128 (64 leave two waves without
+// columns), and for K <= 64, whose short K loop gains more from the third
+// block per CU than from the wider strip (fixed scale 200000 x 64 -> 132 62.6 ->
+// 50.1 us, -> 300 93.5 -> 75.3, -> 512 105 -> 102.5; FP8 and per-token alike).
 template <int FMT>
 static void launch_token_fmt(const RowsArgs& a, int act, hipStream_t st) {
     if (token_small_tiles(a)) return launch_token_rag<FMT, 2, 1>(a, act, st);
-    if (!token_whole(a)) return a.N <= 128 ? launch_token_rag<FMT, 2, 4>(a, act, st) : launch_token_rag<FMT, 4, 4>(a, act, st);
-    if (a.N <= 128) launch_token_whole<FMT, 2>(a, act, st);
+    const bool narrow = a.N <= 128 || a.K <= 64;
+    if (!token_whole(a)) return narrow ? launch_token_rag<FMT, 2, 4>(a, act, st) : launch_token_rag<FMT, 4, 4>(a, act, st);
+    if (narrow) launch_token_whole<FMT, 2>(a, act, st);
     else launch_token_whole<FMT, 4>(a, act, st);
 }
 

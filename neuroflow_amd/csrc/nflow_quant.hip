@@ -650,13 +650,28 @@ static int formula_row(int K) { return K <= 4096 ? F_ROW_VNNI : F_ROW_SCALAR; }
 // (NFLOW_NO_GEMM=1 selects the row-tile kernel instead, for A/B timing).
 static bool use_gemm(const RowsArgs& a) { return gemm_ok(a) && !path_flag(kernel_path().no_gemm); }
 
-// Whether a layer on fp32 input takes the one-pass kernel (token_gemm_kernel.h)
-// rather than the row-tile kernel or the generic one.  The row-tile kernel
-// stays where it can run (weights in registers: 300000 x 64 -> 40 26.9 us
-// either way).
+// Where a layer on fp32 input takes the row-tile kernel (weights in registers
+// or re-read per 16 rows, no barriers) rather than the one-pass kernel.
+// Measured on MI355X (us, row-tile / one-pass):
+//   K, N <= 64: 300000 x 64 -> 40 26.9 either way; it stays;
+//   per-token INT8 of K < 64 into a few more columns, many rows: 200000 x 8 ->
+//     132 42.6 / 61, x 48 -> 68 34.5 / 45, but x 32 -> 256 120 / 70 and
+//     40000 x 4 -> 132 16.6 / 15.6;
+//   FP8 and fixed scale, two K blocks into at most 16 columns, many rows:
+//     150000 x 100 -> 8 24.6 / 29.4 and 26.6 / 31, but 60000 x 80 -> 20 13.9 /
+//     12.8 and 150000 x 100 -> 40 43 / 32.
+static bool use_rows(const RowsArgs& a, int in_mode, bool fp8) {
+    if (!rows_ok(a, in_mode)) return false;
+    if (a.N <= 64 && a.K <= 64) return true;
+    if (path_flag(kernel_path().token_rows)) return false;   // forced tiles: one-pass
+    if (in_mode == IN_F32_TOKEN && !fp8) return a.K < 64 && a.N <= 160 && a.M >= 65536;
+    return a.K > 64 && a.K <= 128 && a.N <= 16 && a.M >= 100000;
+}
+
+// Whether a layer on fp32 input that use_rows does not claim takes the one-pass
+// kernel (token_gemm_kernel.h) rather than the generic one.
 static bool use_token_gemm(const RowsArgs& a) {
-    if (!token_gemm_ok(a) || path_flag(kernel_path().no_token_gemm)) return false;
-    return !rows_ok(a, IN_F32_TOKEN);
+    return token_gemm_ok(a) && !path_flag(kernel_path().no_token_gemm);
 }
 
 // Whether a layer on fp32 input takes the few-row kernel (skinny_kernel.h):
@@ -745,10 +760,18 @@ static int int8_fixed_path(const nflow_int8_linear_params* p, int64_t rows, cons
         launch_rows64_fixed(a, st);
         return check_launch(what);
     }
+    if (use_rows(a, IN_F32_FIXED, false)) {
+        launch_rows<false, IN_F32_FIXED, OUT_EPI>(a, ACT_NONE, st);
+        return check_launch(what);
+    }
     RowsArgs g = a;
     g.Aq = nullptr;  // the codes go to the workspace, which is 256-byte aligned
     const bool wide = aligned(A, 16) && use_gemm(g);
-    if (use_token_gemm(a) && !(wide && fixed_split_faster(a) && !stream_capturing(st))) {
+    // A few dozen products per row, many rows, N off 4: a thread per output on
+    // codes (150000 x 4 -> 5 9.6 us, one-pass 20.9; x 16 -> 3 13.4 / 20.7; at
+    // x 16 -> 5 both 21).
+    const bool tiny = static_cast<int64_t>(a.K) * a.N <= 48 && rows >= 32768;
+    if (use_token_gemm(a) && !((tiny || (wide && fixed_split_faster(a))) && !stream_capturing(st))) {
         launch_token_i8_fixed(a, st);
         return check_launch(what);
     }
@@ -777,11 +800,12 @@ static int int8_fixed_path(const nflow_int8_linear_params* p, int64_t rows, cons
         launch_gemm<OUT_EPI>(a, ACT_NONE, st);
         return check_launch(what);
     }
-    if (rows_ok(a, IN_F32_FIXED)) {
-        launch_rows<false, IN_F32_FIXED, OUT_EPI>(a, ACT_NONE, st);
+    Scratch ws(static_cast<size_t>(rows) * a.K, st);
+    if (ws.err != hipSuccess && use_token_gemm(a)) {
+        (void)hipGetLastError();
+        launch_token_i8_fixed(a, st);
         return check_launch(what);
     }
-    Scratch ws(static_cast<size_t>(rows) * a.K, st);
     if (ws.err != hipSuccess) return set_error(NFLOW_INTERNAL, std::string(what) + ": workspace allocation failed");
     const int64_t n = rows * a.K;
     const int per = elem_per(n, aligned(A, 16));
@@ -1054,6 +1078,10 @@ static int int8_per_token(const nflow_int8_linear_params* p, int64_t M, const fl
         launch_skinny_i8(a, act_x2, st);
         return finish();
     }
+    if (use_rows(a, IN_F32_TOKEN, false)) {
+        launch_rows<false, IN_F32_TOKEN, OUT_EPI>(a, act_x2, st);
+        return finish();
+    }
     // The split form takes a workspace: not where the no-allocation entry
     // point's callers rely on the shape using none, nor for a capture that the
     // one-pass kernel can serve.
@@ -1064,10 +1092,6 @@ static int int8_per_token(const nflow_int8_linear_params* p, int64_t M, const fl
     const bool split = wide && split_faster(a) && !none_taken && (fixed || !stream_capturing(st));
     if (!refused && one_pass && !split) {
         launch_token_i8(a, act_x2, st);
-        return finish();
-    }
-    if (!wide && rows_ok(a, IN_F32_TOKEN)) {
-        launch_rows<false, IN_F32_TOKEN, OUT_EPI>(a, act_x2, st);
         return finish();
     }
     // Split path: quantise into a workspace, then the product.
@@ -1315,6 +1339,10 @@ static int fp8_per_token(const nflow_fp8_linear_params* p, int64_t M, const floa
         launch_skinny_fp8(a, act_x2, st);
         return finish();
     }
+    if (use_rows(a, IN_F32_TOKEN, true)) {
+        launch_rows<true, IN_F32_TOKEN, OUT_EPI>(a, act_x2, st);
+        return finish();
+    }
     // K a multiple of 64, at least 512: quantise, then the tiled GEMM, where
     // that is the faster form.
     RowsArgs g = a;
@@ -1322,10 +1350,6 @@ static int fp8_per_token(const nflow_fp8_linear_params* p, int64_t M, const floa
     const bool wide = a.K >= 512 && use_gemm(g);
     if (use_token_gemm(a) && !(wide && fp8_split_faster(a) && !stream_capturing(st))) {
         launch_token_fp8(a, act_x2, st);
-        return finish();
-    }
-    if (rows_ok(a, IN_F32_TOKEN)) {
-        launch_rows<true, IN_F32_TOKEN, OUT_EPI>(a, act_x2, st);
         return finish();
     }
     const size_t codes = static_cast<size_t>(M) * a.K;

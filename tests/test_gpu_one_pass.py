@@ -234,3 +234,46 @@ def test_whole_shapes(gpu, tile_rows, M, K, N):
         (np.abs(O.e4m3_decode(qw)) * s8[:, None]).astype(np.float64).T
     bound = (K + 3) * 2.0 ** -24 * (terms + np.abs(b)[None, :]) + 1e-38
     assert np.all(np.abs(y.cpu().numpy()[rows].astype(np.float64) - want) <= bound)
+
+
+# Many rows of small layers: the row-tile kernel's share (per-token INT8 of K < 64
+# into 65 to 160 columns, FP8 and fixed scale of 65 <= K <= 128 into at most 16), a
+# thread per output (K N <= 48), and their neighbours on the one-pass kernel.
+@pytest.mark.parametrize("kind,M,K,N", [("int8", 65537, 8, 132), ("int8", 65600, 60, 68), ("int8", 65536, 4, 160),
+                                        ("int8", 65536, 64, 132), ("int8", 65537, 8, 164), ("fp8", 100003, 100, 8),
+                                        ("fp8", 100000, 128, 16), ("fp8", 100000, 68, 20), ("fixed", 100003, 100, 8),
+                                        ("fixed", 100000, 128, 16), ("fixed", 32769, 4, 5), ("fixed", 40001, 16, 3),
+                                        ("fixed", 32769, 7, 7)])
+def test_many_rows_of_small_layers(gpu, kind, M, K, N):
+    base = 1009
+    A = WL.normal(900, (base, K))
+    idx = torch.arange(M, device="cuda") % base
+    x = torch.from_numpy(A).cuda()[idx].contiguous()
+    q, s, zps, sw, b = _int8(N, K, 901)
+    buf, out = _guarded(M, N, 0)
+    st = torch.cuda.current_stream().cuda_stream
+    if kind == "fp8":
+        qw, s8 = O.quantise_weight_fp8(WL.uniform(902, (N, K), -0.125, 0.125))
+        Q.fp8_linear_forward_per_token(Q.Fp8LinearParams(_cu(qw, 0), _cu(s8, 0), _cu(b, 0)), x, "none", out=out)
+        qa, sa = O.quantise_per_token_fp8(A)
+        want = O.layer_fp8_exact(qa, sa, qw, s8, b, 0)
+        terms = (np.abs(O.e4m3_decode(qa)) * sa[:, None]).astype(np.float64) @ \
+            (np.abs(O.e4m3_decode(qw)) * s8[:, None]).astype(np.float64).T
+        bound = (K + 3) * 2.0 ** -24 * (terms + np.abs(b)[None, :]) + 1e-38
+        assert np.all(np.abs(out[:base].cpu().numpy().astype(np.float64) - want) <= bound)
+        assert torch.equal(out.view(torch.int32), out[:base][idx].view(torch.int32))
+    elif kind == "int8":
+        p = Q.Int8LinearParams(_cu(q, 0), _cu(s, 0), _cu(zps, 0), _cu(b, 0), sum_W_per_row=_cu(sw, 0))
+        Q.linear_forward_per_token(p, x, "relu", out=out)
+        want, _ = O.layer_per_token_i8(A, q, s, zps, b, sw, 1)
+        assert torch.equal(out.view(torch.int32), torch.from_numpy(want).cuda()[idx].view(torch.int32))
+    else:
+        ps = Q.Int8LinearParams(_cu(q, 0), _cu(s, 0), _cu(zps, 0), _cu(b, 0), 0.02, 5, _cu(sw, 0))
+        for fn, ref in ((_lib.lib().nflow_int8_linear_forward_batched, O.linear_forward_batched),
+                        (_lib.lib().nflow_int8_linear_forward_rows, O.linear_forward_rows)):
+            out.fill_(7.0)
+            _lib.check(fn(ctypes.byref(ps.c_struct()), M, x.data_ptr(), out.data_ptr(), st), "fixed")
+            rc, want = ref(A, q, s, zps, b, 0.02, 5, sw)
+            assert rc == 0
+            assert torch.equal(out.view(torch.int32), torch.from_numpy(want).cuda()[idx].view(torch.int32))
+    assert _guards_kept(buf, M, N, 0)
