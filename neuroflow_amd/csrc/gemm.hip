@@ -27,19 +27,26 @@ static void launch_gemm_t(const RowsArgs& a, hipStream_t st) {
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(256), lds, st, a, groups);
 }
 
-// Tile shape: 128 x 256 for large M and N (two blocks per CU), else 128 x 128
-// where that gives every CU a block, else 64 x 64 (four times the blocks, and
-// a lone block's K steps take half the time).  Measured on MI355X: 256 x 256
-// (one wave per SIMD) never beats 128 x 256; static 4096 x 1024 -> 256 with its
-// quantise 22.5 us at 128 x 128, 13.9 at 64 x 64.
+// Tile shape: 128 x 256 for large M and N (two blocks per CU); 64 x 64 while
+// there are at most two per CU (a lone block's K steps take half the time);
+// then 128 x 128, but for K < 1024 with at most one per CU (two for K <= 256),
+// where 64 x 128 gives more blocks.  Measured on MI355X (us, 64 x 64 / 64 x 128 / 128 x 128):
+// codes in, int32 out, 4096 x 3072 -> 256 11.5 / 13 / 17, 12000 x 1536 -> 256 (752
+// blocks of 64 x 64) 12.2 / 9.8 / 9.7, 9000 x 2048 -> 384 17.4 / 12.6 / 11.7; a
+// per-token layer with its quantise 2000 x 960 -> 512 14.0 / 15.1 / 17.7, 4096 x
+// 640 -> 768 14.8 / 14.3 / 15.6, 8192 x 640 -> 1024 27.0 / 24.8 / 23.8.  256 x 256
+// (one wave per SIMD) never beats 128 x 256.
 static int gemm_shape(const RowsArgs& a) {
     // A gemm_tile override of 88|48|44|24|22 forces a shape (for tile sweeps;
     // 22 and 24 only on the LDS-DMA kernel).
     const int t = kernel_path().gemm_tile.load(std::memory_order_relaxed);
     if (t == 88 || t == 48 || t == 44 || t == 22 || t == 24) return t;
     if (a.M >= 16384 && a.N >= 1024) return 48;
-    const int64_t blocks = ((a.M + 127) / 128) * ((static_cast<int64_t>(a.N) + 127) / 128);
-    return a.N <= 64 || blocks < num_cus() ? 22 : 44;
+    const int64_t cus = num_cus();
+    const int64_t b64 = ((a.M + 63) / 64) * ((static_cast<int64_t>(a.N) + 63) / 64);
+    if (a.N <= 64 || b64 <= 2 * cus) return 22;
+    const int64_t b128 = ((a.M + 127) / 128) * ((static_cast<int64_t>(a.N) + 127) / 128);
+    return a.K < 1024 && b128 <= (a.K <= 256 ? 2 * cus : cus) ? 24 : 44;
 }
 
 template <int TM, int TN, int OUT, int ACT>
