@@ -697,21 +697,45 @@ static bool use_skinny(const RowsArgs& a) {
 // launch): whether that split is the faster form.  The one-pass kernel reads
 // all the weights once per row tile, the split form reads the activations
 // once and the codes per column block.  Measured on MI355X (us, one-pass /
-// split): K <= 256 one-pass throughout (12000 x 256 -> 1024 18.1 / 20.1, 65536
-// x 192 -> 2048 127 / 161) but for wide rows of part lines (20000 x 256 ->
-// 1000 33.6 / 28.5); larger K at 16-row tiles one-pass (1500 x 320 -> 512 8.8 /
-// 9.8, 3000 x 512 -> 256 10.2 / 10.9); at 64-row tiles split (12000 x 384 ->
-// 1024 29 / 27, 8192 x 512 -> 1024 22 / 17) until there are enough row tiles
-// (20000 x 512 -> 256 19.7 / 22.2, 32768 x 384 -> 2048 83 / 102), and split again
-// at K = 512 with wide N, where the persistent GEMM runs (65536 x 512 -> 768
-// 85 / 73, -> 2048 183 / 145).
+// split) over K = 192 .. 512, 22 row counts from 600 to 100000, 12 widths:
+//   K <= 256: one-pass for whole shapes (20000 x 256 -> 512 17.9 / 20.4).  The
+//     masked form loses to the GEMM at K = 256 (3000 -> 1000 15.4 / 10.8, 20000 ->
+//     300 21.9 / 18.1, 80000 -> 800 92 / 75), at K = 192 with at most three
+//     quarters of a 64-row tile per CU (6000 -> 640 13.8 / 10.5) and where the
+//     last round is half empty (40000 -> 1000 58 / 52), at K = 128 into wide rows
+//     (3000 -> 2000 15.1 / 11.8, 40000 -> 800 47 / 40);
+//   larger K at 16-row tiles: one-pass up to 2.5 (row tile, 128-column chunk)
+//     pairs per CU (2000 x 384 -> 500 9.2 / 9.7, 3000 -> 1000 16.9 / 12.3), 4 with
+//     part lines at K = 512 (2500 x 512 -> 500 12.3 / 13.7), and for narrow N
+//     throughout (8192 x 320 -> 300 11.6 / 13.2);
+//   at 64-row tiles two blocks per CU work through the tiles in rounds: split
+//     with at most a tile per CU (12000 x 384 -> 1024 29 / 27) and where the last
+//     round leaves a third of the slots idle (20000 x 384 -> 300 29.7 / 26.5, 40000
+//     x 320 -> 1000 76 / 64), one-pass elsewhere (32768 x 384 -> 576 36.5 / 45,
+//     65536 x 448 -> 1024 97 / 152);
+//   K = 512, where the persistent GEMM runs: split from N = 1024 (65536 110 / 88)
+//     and from N = 512 beyond one round (65536 x 512 -> 576 74 / 68; 32768 37.5 /
+//     40), one-pass with wide rows of part lines (16384 -> 1000 37.6 / 48).
 static bool split_faster(const RowsArgs& a) {
     if (a.K > 512) return true;
-    if (a.K <= 256) return a.K > 192 && a.N > 512 && a.N % 32 != 0 && a.M < 32768 && !token_small_tiles(a);
-    if (token_small_tiles(a)) return false;
-    if (a.M < 16384) return true;
-    if (a.N <= 256) return false;
-    return a.M < 32768 || (a.K == 512 && a.N > 512 && a.N % 32 == 0);
+    const int64_t cus = num_cus(), tiles = (a.M + 63) / 64;
+    const int64_t pairs = ((a.M + 15) / 16) * ((static_cast<int64_t>(a.N) + 127) / 128);
+    const int64_t slots = 2 * cus, rounds = (tiles + slots - 1) / slots;
+    const int64_t fill = 100 * tiles / (rounds * slots);   // per cent, of the rounds' slots
+    const bool part_lines = a.N % 32 != 0;
+    if (a.K <= 256) {
+        if (token_whole(a)) return false;
+        if (a.K == 256) return a.N > 192 && 2 * pairs > 7 * cus;
+        if (token_small_tiles(a)) return false;
+        return a.K == 128 ? a.N >= 768 : a.N > 256 && (4 * tiles <= 3 * cus || (tiles > slots && fill < 65));
+    }
+    if (token_small_tiles(a))
+        return a.N > (a.K == 512 && !part_lines ? 255 : 384) && 2 * pairs > (a.K == 512 && part_lines ? 8 : 5) * cus;
+    if (tiles < cus) return true;
+    if (a.K < 512) return a.N > 256 && (tiles == cus || fill < 68);
+    if (part_lines) return a.N <= 384 && tiles > cus && tiles <= slots && fill < 65;
+    if (a.N >= 1024 || (a.N >= 512 && tiles > slots)) return true;
+    return a.N > 256 && tiles > cus && fill < 65;
 }
 
 // The same choice for FP8 (K >= 512).  Measured on MI355X (us, one-pass /

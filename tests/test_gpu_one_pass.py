@@ -277,3 +277,32 @@ def test_many_rows_of_small_layers(gpu, kind, M, K, N):
             assert rc == 0
             assert torch.equal(out.view(torch.int32), torch.from_numpy(want).cuda()[idx].view(torch.int32))
     assert _guards_kept(buf, M, N, 0)
+
+
+# Sizes on both sides of the rules that choose between the one-pass kernel and
+# quantise + GEMM, and among the GEMM's tiles; whichever runs, the same bits.
+@pytest.mark.parametrize("M,K,N", [(3000, 128, 800), (1000, 128, 800), (3000, 256, 1000), (1500, 256, 1000), (6000, 192, 640),
+                                   (12500, 192, 640), (2000, 384, 1000), (1000, 384, 1000), (4096, 512, 500), (16385, 320, 300),
+                                   (4096, 640, 768), (9000, 1536, 384), (2100, 960, 516), (300, 3072, 512)])
+def test_same_bits_in_either_form(gpu, M, K, N):
+    base = 997
+    q, s, zps, sw, b = _int8(N, K, 920)
+    A = WL.normal(923, (base, K))
+    idx = torch.arange(M, device="cuda") % base
+    x = torch.from_numpy(A).cuda()[idx].contiguous()
+    p = Q.Int8LinearParams(_cu(q, 0), _cu(s, 0), _cu(zps, 0), _cu(b, 0), sum_W_per_row=_cu(sw, 0))
+    want, _ = O.layer_per_token_i8(A[:min(M, base)], q, s, zps, b, sw, 1)
+    want = torch.from_numpy(want).cuda()[idx]
+    L = _lib.lib()
+    for path in (None, b"no_gemm", b"no_token_gemm"):
+        if path == b"no_gemm" and K > 1024:
+            continue     # that leaves the generic kernel
+        prev = ctypes.c_int(0)
+        if path:
+            _lib.check(L.nflow_debug_set_kernel_path(path, 1, ctypes.byref(prev)), "path")
+        try:
+            y = Q.linear_forward_per_token(p, x, "relu")
+        finally:
+            if path:
+                _lib.check(L.nflow_debug_set_kernel_path(path, prev.value, None), "path")
+        assert torch.equal(y.view(torch.int32), want.view(torch.int32)), path
