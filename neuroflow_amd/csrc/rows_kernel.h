@@ -488,7 +488,11 @@ __global__ __launch_bounds__(256, rows_min_waves(KB, FP8)) void k_rows(RowsArgs 
 #pragma unroll
                     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) xc[kb][j] = pack4_token_exact(cur.x[kb][j], srow, inv);
+                        for (int j = 0; j < 4; ++j) {
+                            xc[kb][j] = pack4_token_exact(cur.x[kb][j], srow, inv);
+                            // 0 / 0 past K in a row whose scale rounds to 0.
+                            if (!KFULL && kb * 64 + j * 16 + g * 4 >= K) xc[kb][j] = 0u;
+                        }
                 }
             } else {
 #pragma unroll

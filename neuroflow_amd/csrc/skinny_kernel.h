@@ -168,6 +168,7 @@ __global__ __launch_bounds__(64 * NW) void k_skinny(RowsArgs a) {
                 Sf += ws_s[w][c];
                 Sd += wd_s[w][c];
             }
+            if constexpr (FMT == TG_I8_TOKEN) SA += token_sum_past_k(scale_s[rr], 64 * NW * PER - K);
             const IntEpi e = int_epi_consts(a.formula, K, a.zp_A, a.zpW ? a.zpW[col] : 0, a.sumW ? a.sumW[col] : 0,
                                             a.sumW != nullptr, Sf, Sd);
             tv = int_epi_value_of<FMT == TG_I8_FIXED>(e, D, SA);

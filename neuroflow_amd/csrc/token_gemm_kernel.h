@@ -135,6 +135,11 @@ __device__ __forceinline__ uint32_t token_mask_codes(uint32_t v, int left) {
     return left <= 0 ? 0u : (left < 4 ? v & ((1u << (8 * left)) - 1u) : v);
 }
 
+// Per-token INT8 codes past K are 0 (and meet weights of 0) except in a row
+// whose scale rounded to 0: there every code is that of x / 0 or 0 / 0, -128, and
+// the row's code sum takes back the ones past K.
+__device__ __forceinline__ int32_t token_sum_past_k(float s, int past) { return s == 0.0f ? 128 * past : 0; }
+
 // Codes of local row lr (= 4 q + g of the wave's rows) from x into the tile
 // and, for INT8, their byte sum; row scale and sum to lds_s / lds_sa (and
 // the per-token scale to scale_out for rows < M).
@@ -187,6 +192,7 @@ __device__ __forceinline__ void token_quantise_row(const RowsArgs& a, const v4f 
         sa += dpp_movi<0x4E>(sa);
         sa += dpp_movi<0x141>(sa);
         sa += dpp_movi<0x140>(sa);
+        if constexpr (RAG && FMT == TG_I8_TOKEN) sa += token_sum_past_k(s, 64 * J - a.K);
     }
     if (r == 0) {
         lds_s[lr] = s;

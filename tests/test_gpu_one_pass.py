@@ -306,3 +306,26 @@ def test_same_bits_in_either_form(gpu, M, K, N):
             if path:
                 _lib.check(L.nflow_debug_set_kernel_path(path, prev.value, None), "path")
         assert torch.equal(y.view(torch.int32), want.view(torch.int32)), path
+
+
+@pytest.mark.parametrize("M,K,N,path", [(70, 100, 65, None), (70, 60, 260, None), (33, 1000, 36, None), (40, 20, 36, None),
+                                        (5, 100, 48, "skinny"), (3, 1000, 20, "skinny")])
+def test_rows_of_vanishing_scale(gpu, M, K, N, path):
+    """Rows so small that absmax / 127 rounds to 0: every code is -128 and the
+    output is the bias plus a zero whose sign is the integer result's, so a
+    code past K in the row's sum shows under a bias of -0."""
+    q, s, zps, sw, _ = _int8(N, K, 910)
+    b = np.full(N, -0.0, np.float32)
+    A = np.full((M, K), 1e-44, np.float32)
+    A[1::2, ::3] = -7e-45
+    L = _lib.lib()
+    prev = ctypes.c_int(0)
+    if path:
+        _lib.check(L.nflow_debug_set_kernel_path(path.encode(), 1, ctypes.byref(prev)), "path")
+    p = Q.Int8LinearParams(_cu(q, 0), _cu(s, 0), _cu(zps, 0), _cu(b, 0), sum_W_per_row=_cu(sw, 0))
+    got = Q.linear_forward_per_token(p, _cu(A, 0), "none").cpu().numpy()
+    if path:
+        _lib.check(L.nflow_debug_set_kernel_path(path.encode(), prev.value, None), "path")
+    want, sc = O.layer_per_token_i8(A, q, s, zps, b, sw, 0)
+    assert (sc == 0.0).all() and np.signbit(want).any() and not np.signbit(want).all()
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
