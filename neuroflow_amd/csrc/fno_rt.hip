@@ -233,6 +233,12 @@ __global__ __launch_bounds__(256) void k_linear_k1(LinArgs a) {
 // 32: 473 us).  Row r of the launch is output row r; its input row and
 // validity follow LinArgs.
 constexpr int kLinRows = 8;
+// Fewer rows leave most CUs without a block, and the few that run stage all
+// of W for 32 rows each: one thread per output is then shorter (FNO1d of 3
+// layers without quantisation, us, per output / blocked: width 128, 64 rows
+// 144 / 242, 1024 rows 228 / 284, 2048 rows 341 / 263; width 96, 1024 rows
+// 186 / 216, 2048 rows 225 / 210; width 56, 1024 rows 109 / 115, 2048 129 / 110).
+constexpr int64_t kLinBlockRows = 1536;
 constexpr int lin_block_rows(int cw) { return 4 * (64 / cw) * kLinRows; }
 inline size_t lin_block_lds(int k, int cw) {
     const size_t ks = (static_cast<size_t>(k) + 3) / 4 * 4;
@@ -1649,7 +1655,7 @@ hipError_t launch_linear_ref(const LinArgs& a, hipStream_t st) {
     } else if (a.k == 1 && a.rows_in == a.rows_out && a.rows_valid == a.rows_out && a.n >= 4 && a.n <= 1024 &&
                (a.n & (a.n - 1)) == 0 && aligned(a.y, 16)) {
         hipLaunchKernelGGL(k_linear_k1, dim3(grid_for(rows * (a.n / 4), 256, 8)), dim3(256), 0, st, a);
-    } else if (lin_block_lds(a.k, a.n > 32 ? 64 : 32) <= 64 * 1024) {
+    } else if (rows >= kLinBlockRows && lin_block_lds(a.k, a.n > 32 ? 64 : 32) <= 64 * 1024) {
         if (a.n > 32) launch_linear_block<64>(a, rows, st);
         else launch_linear_block<32>(a, rows, st);
     } else {

@@ -80,3 +80,18 @@ def test_blocked_linear(gpu, tmp_path, case):
     y = _run(tmp_path, ir, x, case[3])
     want = OF.forward(m, x)
     assert np.array_equal(T1._bits(y), T1._bits(want))
+
+
+# The same forms at the row counts the blocked Linear serves (1536 and more;
+# the cases above run one thread per output).
+@pytest.mark.parametrize("case", [(48, 32, 2, 1, 17, 6, 2, 1, False, None, False),
+                                  (201, 8, 3, 2, 33, 4, 1, 1, True, ["tensor"], False),
+                                  (99, 16, 1, 1, 70, 4, 1, 1, False, ["fp8"], False),
+                                  (400, 4, 3, 1, 20, 2, 2, 8, False, ["tensor"], False),
+                                  (8, 256, 1, 1, 100, 4, 1, 1, False, None, False),
+                                  (6, 256, 1, 1, 28, 4, 2, 1, False, None, False)], ids=T1._ids)
+def test_blocked_linear_many_rows(gpu, tmp_path, case):
+    ir, x, m = T1._model(case)
+    y = _run(tmp_path, ir, x, case[3])
+    want = OF.forward(m, x)
+    assert np.array_equal(T1._bits(y), T1._bits(want))
