@@ -28,14 +28,17 @@ static void launch_gemm_t(const RowsArgs& a, hipStream_t st) {
 }
 
 // Tile shape: 128 x 256 for large M and N (two blocks per CU); 64 x 64 while
-// there are at most two per CU (a lone block's K steps take half the time);
-// then 128 x 128, but for K < 1024 with at most one per CU (two for K <= 256),
-// where 64 x 128 gives more blocks.  Measured on MI355X (us, 64 x 64 / 64 x 128 / 128 x 128):
-// codes in, int32 out, 4096 x 3072 -> 256 11.5 / 13 / 17, 12000 x 1536 -> 256 (752
-// blocks of 64 x 64) 12.2 / 9.8 / 9.7, 9000 x 2048 -> 384 17.4 / 12.6 / 11.7; a
-// per-token layer with its quantise 2000 x 960 -> 512 14.0 / 15.1 / 17.7, 4096 x
-// 640 -> 768 14.8 / 14.3 / 15.6, 8192 x 640 -> 1024 27.0 / 24.8 / 23.8.  256 x 256
-// (one wave per SIMD) never beats 128 x 256.
+// there are at most two per CU (a lone block's K steps take half the time), two
+// and a half where the epilogue has integer terms; then 128 x 128, but with at
+// most one per CU (two for K <= 256) 64 x 128, which gives more blocks, where K <
+// 1024 or the epilogue has terms.  Measured on MI355X (us, 64 x 64 / 64 x 128 /
+// 128 x 128): codes in, int32 out, 4096 x 3072 -> 256 8.5 / 9.9 / 14.4, 12000 x
+// 1536 -> 256 (752 blocks of 64 x 64) 12.2 / 9.8 / 9.7, 9000 x 2048 -> 384 17.4 /
+// 12.6 / 11.7; a symmetric per-token layer with its quantise 2000 x 960 -> 512
+// 14.0 / 15.1 / 17.7, 4096 x 640 -> 768 14.8 / 14.3 / 15.6, 8192 x 640 -> 1024 27.0 /
+// 24.8 / 23.8; fixed scale with zero points 9000 x 1536 -> 256 (564) 30.4 / 31.6 /
+// 32.9, 4096 x 2048 -> 928 31.6 / 28.3 / 29.3.  256 x 256 (one wave per SIMD) never
+// beats 128 x 256.
 static int gemm_shape(const RowsArgs& a) {
     // A gemm_tile override of 88|48|44|24|22 forces a shape (for tile sweeps;
     // 22 and 24 only on the LDS-DMA kernel).
@@ -43,10 +46,11 @@ static int gemm_shape(const RowsArgs& a) {
     if (t == 88 || t == 48 || t == 44 || t == 22 || t == 24) return t;
     if (a.M >= 16384 && a.N >= 1024) return 48;
     const int64_t cus = num_cus();
+    const bool terms = a.zpW || a.zp_A != 0 || (a.formula == F_ROW_VNNI && a.sumW);
     const int64_t b64 = ((a.M + 63) / 64) * ((static_cast<int64_t>(a.N) + 63) / 64);
-    if (a.N <= 64 || b64 <= 2 * cus) return 22;
+    if (a.N <= 64 || 2 * b64 <= (terms ? 5 : 4) * cus) return 22;
     const int64_t b128 = ((a.M + 127) / 128) * ((static_cast<int64_t>(a.N) + 127) / 128);
-    return a.K < 1024 && b128 <= (a.K <= 256 ? 2 * cus : cus) ? 24 : 44;
+    return (a.K < 1024 || terms) && b128 <= (a.K <= 256 ? 2 * cus : cus) ? 24 : 44;
 }
 
 template <int TM, int TN, int OUT, int ACT>
