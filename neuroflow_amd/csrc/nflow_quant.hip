@@ -657,15 +657,18 @@ static bool use_gemm(const RowsArgs& a) { return gemm_ok(a) && !path_flag(kernel
 //   per-token INT8 of K < 64 into a few more columns, many rows: 200000 x 8 ->
 //     132 42.6 / 61, x 48 -> 68 34.5 / 45, but x 32 -> 256 120 / 70 and
 //     40000 x 4 -> 132 16.6 / 15.6;
-//   FP8 and fixed scale, two K blocks into at most 16 columns, many rows:
-//     150000 x 100 -> 8 24.6 / 29.4 and 26.6 / 31, but 60000 x 80 -> 20 13.9 /
-//     12.8 and 150000 x 100 -> 40 43 / 32.
+//   two K blocks into few columns, many rows: FP8 into 16 and fewer 30000 x 100
+//     -> 16 7.3 / 8.6, 60000 10.4 / 14.0, but -> 20 14.0 / 14.2; fixed scale 60000 x 100
+//     -> 20 12.4 / 15.4, -> 40 16.5 / 17.0, x 128 -> 20 15.2 / 15.8; per-token INT8
+//     60000 x 100 -> 20 10.6 / 17.5, 350000 -> 48 64 / 80, x 128 -> 20 12.1 / 15.4, but
+//     100000 x 128 -> 32 24.7 / 23.8 and 30000 x 128 -> 20 8.4 / 8.1.
 static bool use_rows(const RowsArgs& a, int in_mode, bool fp8) {
     if (!rows_ok(a, in_mode)) return false;
     if (a.N <= 64 && a.K <= 64) return true;
     if (path_flag(kernel_path().token_rows)) return false;   // forced tiles: one-pass
-    if (in_mode == IN_F32_TOKEN && !fp8) return a.K < 64 && a.N <= 160 && a.M >= 65536;
-    return a.K > 64 && a.K <= 128 && a.N <= 16 && a.M >= 100000;
+    if (a.K > 64 && fp8) return a.N <= 16 && a.M >= 24576;
+    if (a.K > 64) return a.N <= (a.K == 128 ? 20 : in_mode == IN_F32_TOKEN ? 48 : 40) && a.M >= 49152;
+    return in_mode == IN_F32_TOKEN && !fp8 && a.K < 64 && a.N <= 160 && a.M >= 65536;
 }
 
 // Whether a layer on fp32 input that use_rows does not claim takes the one-pass

@@ -237,12 +237,14 @@ def test_whole_shapes(gpu, tile_rows, M, K, N):
 
 
 # Many rows of small layers: the row-tile kernel's share (per-token INT8 of K < 64
-# into 65 to 160 columns, FP8 and fixed scale of 65 <= K <= 128 into at most 16), a
-# thread per output (K N <= 48), and their neighbours on the one-pass kernel.
+# into 65 to 160 columns, two K blocks into a few), a thread per output (K N <=
+# 48), and their neighbours on the one-pass kernel.
 @pytest.mark.parametrize("kind,M,K,N", [("int8", 65537, 8, 132), ("int8", 65600, 60, 68), ("int8", 65536, 4, 160),
                                         ("int8", 65536, 64, 132), ("int8", 65537, 8, 164), ("fp8", 100003, 100, 8),
-                                        ("fp8", 100000, 128, 16), ("fp8", 100000, 68, 20), ("fixed", 100003, 100, 8),
-                                        ("fixed", 100000, 128, 16), ("fixed", 32769, 4, 5), ("fixed", 40001, 16, 3),
+                                        ("fp8", 100000, 128, 16), ("fp8", 100000, 68, 20), ("fp8", 24577, 84, 4),
+                                        ("int8", 49153, 100, 40), ("int8", 49152, 128, 20), ("int8", 49153, 68, 4),
+                                        ("int8", 49160, 72, 48), ("int8", 49160, 72, 52), ("fixed", 100003, 100, 8),
+                                        ("fixed", 100000, 128, 16), ("fixed", 49153, 124, 40), ("fixed", 49153, 128, 24), ("fixed", 32769, 4, 5), ("fixed", 40001, 16, 3),
                                         ("fixed", 32769, 7, 7)])
 def test_many_rows_of_small_layers(gpu, kind, M, K, N):
     base = 1009
