@@ -101,20 +101,26 @@ const char* nflow_last_error(void);
 /* Kernel-path override for A/B timing and for tests that pin one of two
  * kernels computing the same bits (no counterpart in the reference, whose
  * SIMD path is fixed at compile time, int8_gemm.cpp:34-45).  Names:
- * "no_gemm", "no_rows64", "no_token_gemm", "gemm_reg" (0 / 1) and
- * "gemm_tile" (0 = the launcher's choice, else 88, 48, 44, 24 or 22) and
- * "gemm_mfma" (0 = the launcher's choice, else 16 or 32: the MFMA shape of
- * the LDS-DMA GEMM), "no_wide" (0 / 1: keep K = 512 / 1024 layers off the
- * persistent GEMM), "no_rows64_queue" (0 / 1: the K = N = 64 layer with
- * its static tile deal instead of the per-CU tile queue) and
- * "no_layer_tail" (0 / 1: the FNO runtime's width-64 local-linear layer and
- * its tail as two launches instead of one, and its projection head as two
- * to four instead of one) and "generic_fft" (0 / 1: the
- * FNO runtime's row FFTs of 64 .. 1024 points and its channel mix of up to
- * 64 channels on the any-size kernels instead of the fixed-size ones).  The
- * environment variables NFLOW_<NAME> set the initial values, read once at
- * the library's first launch.  Process-wide; *previous (if not NULL)
- * receives the value replaced.  Unknown names return NFLOW_INVALID_ARG. */
+ *   "no_gemm", "no_rows64", "no_token_gemm", "no_wide", "gemm_reg" (0 / 1): the
+ *     tiled GEMMs, the K = N = 64 layer, the one-pass layer, the persistent GEMM
+ *     of K = 512 / 1024 and the LDS-DMA GEMM not taken;
+ *   "gemm_tile" (0 = the launcher's choice, else 88, 48, 44, 24 or 22) and
+ *     "gemm_mfma" (0, 16 or 32): the tiled GEMM's tile and MFMA shape;
+ *   "token_rows" (0 = the launcher's choice, else 16 or 64): rows per tile of
+ *     the one-pass layer;
+ *   "skinny" (0 = the launcher's choice, 1 wherever it can run, 2 never): the
+ *     few-row layer;
+ *   "no_rows64_queue" (0 / 1): the K = N = 64 layer with its static tile deal
+ *     instead of the per-CU tile queue;
+ *   "no_layer_tail" (0 / 1): the FNO runtime's local-linear layer and its tail
+ *     as two launches instead of one, its projection head as two to four;
+ *   "generic_fft" (0 / 1): the FNO runtime's row FFTs of 64 .. 1024 points and
+ *     its channel mix of up to 64 channels on the any-size kernels;
+ *   "no_workspace" (0 / 1): every workspace allocation reports failure.
+ * The environment variables NFLOW_<NAME> set the initial values of all but
+ * token_rows, skinny and no_workspace, read once at the library's first
+ * launch.  Process-wide; *previous (if not NULL) receives the value replaced.
+ * Unknown names return NFLOW_INVALID_ARG. */
 int nflow_debug_set_kernel_path(const char* name, int value, int* previous);
 
 /* ---- nflow-quant kernel API (cpp/include/neuroflow/int8_gemm.h) ------------ */

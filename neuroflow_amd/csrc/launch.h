@@ -60,6 +60,7 @@ struct KernelPath {
     std::atomic<int> no_wide{0};
     std::atomic<int> no_rows64_queue{0};
     std::atomic<int> no_layer_tail{0};   // the FNO runtime's layer + tail and projection head unfused
+    std::atomic<int> no_workspace{0};    // every workspace allocation reports failure (for tests of that route)
     std::atomic<int> generic_fft{0};     // the FNO runtime's row FFTs and channel mix on the any-size kernels
 };
 KernelPath& kernel_path();

@@ -598,6 +598,10 @@ struct Scratch {
     bool owned = false;                    // per-call allocation (freed here)
     std::unique_lock<std::mutex> lock;
     Scratch(size_t bytes, hipStream_t s, int slot = 0) : st(s) {
+        if (path_flag(kernel_path().no_workspace)) {
+            err = hipErrorOutOfMemory;
+            return;
+        }
         bytes = std::max<size_t>(bytes, 256);
         int dev = 0;
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -878,6 +882,7 @@ int nflow_debug_set_kernel_path(const char* name, int value, int* previous) {
                         : n == "no_wide" ? &k.no_wide
                         : n == "no_rows64_queue" ? &k.no_rows64_queue
                         : n == "no_layer_tail" ? &k.no_layer_tail
+                        : n == "no_workspace" ? &k.no_workspace
                         : n == "generic_fft" ? &k.generic_fft : nullptr;
     if (!f) return set_error(NFLOW_INVALID_ARG, "debug_set_kernel_path: unknown name " + n);
     const int old = f->exchange(value, std::memory_order_relaxed);

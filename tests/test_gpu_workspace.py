@@ -116,3 +116,59 @@ def test_host_threads_share_one_stream(gpu):
     for i in range(4):
         for r in range(6):
             assert torch.equal(_bits(outs[i][r]), _bits(want[i]))
+
+
+@pytest.fixture
+def no_workspace():
+    prev = ctypes.c_int(0)
+    L = _lib.lib()
+    _lib.check(L.nflow_debug_set_kernel_path(b"no_workspace", 1, ctypes.byref(prev)), "path")
+    yield L
+    _lib.check(L.nflow_debug_set_kernel_path(b"no_workspace", prev.value, None), "path")
+
+
+def _plain_call(L, kind, M, k, n, sid):
+    """(call(out), M x n) of one layer through the C entry point."""
+    W, b = WL.uniform(sid, (n, k), -0.125, 0.125), WL.uniform(sid + 1, (n,), -0.1, 0.1)
+    cu = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    if kind == "fp8":
+        qw, sw = O.quantise_weight_fp8(W)
+        p = Q.Fp8LinearParams(cu(qw), cu(sw), cu(b))
+        fn, args = L.nflow_fp8_linear_forward_per_token, (None, 1)
+    else:
+        s = O.per_channel_scales(W, 127.0)
+        q, _ = O.quantise_weight_2d(W, s, np.zeros(n, np.int32))
+        p = Q.Int8LinearParams(cu(q), cu(s), cu(np.zeros(n, np.int32)), cu(b), 0.02, 3)
+        fn, args = ((L.nflow_int8_linear_forward_per_token, (None, 1)) if kind == "int8"
+                    else (L.nflow_int8_linear_forward_batched, ()))
+    ps = p.c_struct()
+    x = cu(WL.normal(sid + 2, (M, k)))
+    return lambda out: fn(ctypes.byref(ps), M, x.data_ptr(), out.data_ptr(), *args, torch.cuda.current_stream().cuda_stream), p
+
+
+@pytest.mark.parametrize("kind,M,k,n", [("int8", 4096, 1024, 512), ("int8", 8192, 512, 1024), ("fp8", 4096, 1024, 512),
+                                        ("fixed", 4096, 1024, 512), ("fixed", 40001, 16, 3)])
+def test_failed_workspace_falls_back_to_the_one_pass_kernel(gpu, no_workspace, kind, M, k, n):
+    """Layers the one-pass kernel can serve run there when their workspace
+    cannot be had, with the bits it gives by itself."""
+    L = no_workspace
+    call, keep = _plain_call(L, kind, M, k, n, 770)
+    got, want = torch.full((M, n), float("nan"), device="cuda"), torch.empty(M, n, device="cuda")
+    _lib.check(call(got), kind)
+    prev = ctypes.c_int(0)
+    _lib.check(L.nflow_debug_set_kernel_path(b"no_gemm", 1, ctypes.byref(prev)), "path")
+    try:
+        _lib.check(call(want), kind)
+    finally:
+        _lib.check(L.nflow_debug_set_kernel_path(b"no_gemm", prev.value, None), "path")
+    assert torch.equal(_bits(got), _bits(want))
+
+
+@pytest.mark.parametrize("kind", ["int8", "fp8", "fixed"])
+def test_failed_workspace_is_an_error_beyond_it(gpu, no_workspace, kind):
+    call, keep = _plain_call(no_workspace, kind, 3000, 2048, 256, 780)
+    out = torch.full((3000, 256), 7.0, device="cuda")
+    assert call(out) == _lib.INTERNAL
+    assert b"workspace" in no_workspace.nflow_last_error()
+    torch.cuda.synchronize()
+    assert bool((out == 7.0).all())
