@@ -712,8 +712,9 @@ static bool use_skinny(const RowsArgs& a) {
 //     last round is half empty (40000 -> 1000 58 / 52), at K = 128 into wide rows
 //     (3000 -> 2000 15.1 / 11.8, 40000 -> 800 47 / 40);
 //   larger K at 16-row tiles: one-pass up to 2.5 (row tile, 128-column chunk)
-//     pairs per CU (2000 x 384 -> 500 9.2 / 9.7, 3000 -> 1000 16.9 / 12.3), 4 with
-//     part lines at K = 512 (2500 x 512 -> 500 12.3 / 13.7), and for narrow N
+//     pairs per CU (2000 x 384 -> 500 9.2 / 9.7, 3000 -> 1000 16.9 / 12.3), 3.5 with
+//     part lines at K = 512 (2500 x 512 -> 500 12.3 / 13.7, 2000 -> 1000 15.2 /
+//     14.1), and for narrow N
 //     throughout (8192 x 320 -> 300 11.6 / 13.2);
 //   at 64-row tiles two blocks per CU work through the tiles in rounds: split
 //     with at most a tile per CU (12000 x 384 -> 1024 29 / 27) and where the last
@@ -737,7 +738,7 @@ static bool split_faster(const RowsArgs& a) {
         return a.K == 128 ? a.N >= 768 : a.N > 256 && (4 * tiles <= 3 * cus || (tiles > slots && fill < 65));
     }
     if (token_small_tiles(a))
-        return a.N > (a.K == 512 && !part_lines ? 255 : 384) && 2 * pairs > (a.K == 512 && part_lines ? 8 : 5) * cus;
+        return a.N > (a.K == 512 && !part_lines ? 255 : 384) && 2 * pairs > (a.K == 512 && part_lines ? 7 : 5) * cus;
     if (tiles < cus) return true;
     if (a.K < 512) return a.N > 256 && (tiles == cus || fill < 68);
     if (part_lines) return a.N <= 384 && tiles > cus && tiles <= slots && fill < 65;
@@ -754,15 +755,14 @@ static bool fp8_split_faster(const RowsArgs& a) {
     return a.K > 512 || (a.N > 1024 && !token_small_tiles(a));
 }
 
-// The same choice for fixed-scale INT8.  Measured on MI355X (us, one-pass /
-// split): K = 320 16384 -> 256 18.2 / 22.6, -> 1024 41.1 / 40.5; K = 512, where
-// the split runs the persistent GEMM, 1000 -> 512 9.9 / 10.8, 4096 -> 256 11.8 /
-// 12.1, -> 512 16.2 / 12.5, 8192 -> 2048 41.6 / 30.2, 65536 -> 256 55.4 / 58.6;
-// K = 1024 300 -> 256 13.6 / 11.6, 4096 -> 1024 44 / 17.4, 16384 -> 1024 150 / 45.
+// The same choice for fixed-scale INT8: one-pass for K <= 256, else as per token.
+// Measured on MI355X (us, one-pass / split): 2000 x 320 -> 1024 12.4 / 9.5, 8192 ->
+// 512 15.9 / 13.9; K = 512, 32768 -> 512 33.1 / 40.1, 8192 -> 2048 41.6 / 30.2; K =
+// 1024 300 -> 256 13.6 / 11.6, 16384 -> 1024 150 / 45; at worst, with one tile per CU,
+// 16384 x 320 -> 1024 28.2 / 33.3.
 static bool fixed_split_faster(const RowsArgs& a) {
     if (kernel_path().token_rows.load(std::memory_order_relaxed)) return false;   // forced tiles: one-pass
-    const int64_t pairs = ((a.M + 15) / 16) * ((static_cast<int64_t>(a.N) + 127) / 128);
-    return a.K > 512 || (a.K == 512 && a.N >= 512 && pairs > 2 * static_cast<int64_t>(num_cus()));
+    return a.K > 256 && split_faster(a);
 }
 
 // Fixed-scale int8 path shared by LinearForward / rows / batched.
