@@ -156,31 +156,31 @@ struct PostArgs {
 hipError_t launch_post(const PostArgs& a, hipStream_t st);
 
 // The INT8 local-linear layer (LinearForwardBatched + bias, int8_gemm.cpp:530-580,
-// as fno.cpp:529-536 runs it) and the layer tail in one pass at width 64:
-// x2 = (sW * sA) * D + b from the codes of h quantised with the per-tensor
-// scale sA / zero point zpA, then the tail of PostArgs (p.x2 unused), h
+// as fno.cpp:529-536 runs it) and the layer tail in one pass, at width 64 and
+// the widths of fno_tail.hip: x2 = (sW * sA) * D + b from the codes of h
+// quantised with the per-tensor scale sA / zero point zpA, then the tail of PostArgs (p.x2 unused), h
 // overwritten in place.  Taken when layer_tail_ok holds; the unfused pair
 // computes the same bits.
 struct LayerTailArgs {
     PostArgs p;
-    const int8_t* W;         // (64, 64) codes, row per output channel
-    const float* sW;         // (64)
-    const float* bias;       // (64) or null
-    const int32_t* zpW;      // (64) or null
-    const int32_t* sumW;     // (64) or null
+    const int8_t* W;         // (w, w) codes, row per output channel
+    const float* sW;         // (w)
+    const float* bias;       // (w) or null
+    const int32_t* zpW;      // (w) or null
+    const int32_t* sumW;     // (w) or null
     float sA;
     int32_t zpA;
 };
 bool layer_tail_ok(const PostArgs& p, int in_features, int out_features);
-// The fp32 local linear (64 x 64, launch_linear_ref's sums) and the tail in
-// one pass, on the same conditions; W (64, 64) and b (64 or null) fp32.
+// The fp32 local linear (w x w, launch_linear_ref's sums) and the tail in one
+// pass, on the same conditions; W (w, w) and b (w or null) fp32.
 bool linear_tail_ok(const PostArgs& p, const float* W);
 hipError_t launch_linear_tail(const PostArgs& a, const float* W, const float* b, hipStream_t st);
 
 // The projection head (fno.cpp:662-698, :966-993) in one pass: y = fq_o(
-// proj_out(act(fq_q(proj_q(h))))) for width 64 and one output channel, with
-// the sums and forms of launch_linear_ref and launch_fq_act.  h is
-// token-major with rows_in rows per sample, of which the first n are read;
+// proj_out(act(fq_q(proj_q(h))))) for one output channel, at width 64 and the
+// widths of fno_tail.hip, with the sums and forms of launch_linear_ref and
+// launch_fq_act.  h is token-major with rows_in rows per sample, of which the first n are read;
 // y is (samples, n).
 struct ProjArgs {
     const float* h;

@@ -102,13 +102,7 @@ __global__ __launch_bounds__(256) void k_linear_tail_w(PostArgs a, const float* 
             if (S::TT % S::RP != 0 && t >= S::TT) continue;
             if (!live) continue;
             const float acc = tail_dot<W>(th + t * S::HS, wr, bj);
-            float ps = 0.0f, pz = 0.0f;
-            if constexpr (KIND == 2) {
-                const int64_t p = static_cast<int64_t>(ck) * n + tl.t0 + t;
-                ps = a.pos_scales[p];
-                pz = static_cast<float>(a.pos_zps[p]);
-            }
-            v[q] = post_element<KIND, ACT, FQN>(tx1[ck][t], acc, a, inv_x2, inv_next, thr_x2, thr_next, ps, pz);
+            v[q] = post_element<KIND, ACT, FQN>(tx1[ck][t], acc, a, inv_x2, inv_next, thr_x2, thr_next, 0.0f, 0.0f);
             tx1[ck][t] = v[q];
         }
 #pragma unroll
@@ -282,9 +276,11 @@ __global__ __launch_bounds__(256) void k_proj_tail_w(ProjArgs a) {
     }
 }
 
-// Widths with an instantiation: the multiples of 8 below 64 and 20 (others
-// keep the separate launches).  The rest of the conditions are the width-64
-// forms': whole 32-token tiles, the runtime's activations and fake-quants.
+// Widths with an instantiation: 16 to 48 in steps of 8, and 20.  The kernels
+// hold for any multiple of 4 below 64; the others have not been instantiated or
+// measured and keep the separate launches, as does the per-position x2
+// fake-quant (KIND 2) at every width but 64.  The rest of the conditions are
+// the width-64 forms': whole 32-token tiles, ReLU or GELU, the fake-quants.
 static bool width_ok(int w) { return w == 16 || w == 20 || w == 24 || w == 32 || w == 40 || w == 48; }
 
 bool linear_tail_w_ok(const PostArgs& p, const float* W) {
