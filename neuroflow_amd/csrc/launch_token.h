@@ -33,10 +33,8 @@ static void launch_token_act(const RowsArgs& a, int act, hipStream_t st) {
 
 template <int FMT, int CT, int RT>
 static void launch_token_rag(const RowsArgs& a, int act, hipStream_t st) {
-    if constexpr (CT == 2) {
-        if (a.K <= 64) return launch_token_act<1, FMT, CT, RT, true>(a, act, st);
-    }
-    if (a.K <= 128) launch_token_act<2, FMT, CT, RT, true>(a, act, st);
+    if (a.K <= 64) launch_token_act<1, FMT, CT, RT, true>(a, act, st);
+    else if (a.K <= 128) launch_token_act<2, FMT, CT, RT, true>(a, act, st);
     else if (a.K <= 256) launch_token_act<4, FMT, CT, RT, true>(a, act, st);
     else if (RT == 4 || a.K <= 512) launch_token_act<8, FMT, CT, RT, true>(a, act, st);
     else if constexpr (RT == 1) launch_token_act<16, FMT, CT, RT, true>(a, act, st);
@@ -50,13 +48,15 @@ static void launch_token_whole(const RowsArgs& a, int act, hipStream_t st) {
 }
 
 // 64-row tiles: 32 columns per wave for N <= 128 (64 leave two waves without
-// columns), and for K <= 64, whose short K loop gains more from the third
-// block per CU than from the wider strip (fixed scale 200000 x 64 -> 132 62.6 ->
-// 50.1 us, -> 300 93.5 -> 75.3, -> 512 105 -> 102.5; FP8 and per-token alike).
+// columns), and for K <= 64 up to N = 512, where the short K loop gains more from
+// the third block per CU than from the wider strip (us, 64 columns / 32: fixed
+// scale 200000 x 64 -> 132 62.6 / 50.1, -> 300 93.5 / 75.3, 40000 -> 512 29.0 / 22.1;
+// FP8 and per-token alike; FP8 53783 x 48 -> 512, whose tiles just pass a round
+// of three blocks, 28.4 / 32.8; wider, FP8 23854 x 64 -> 1268 84 / 94).
 template <int FMT>
 static void launch_token_fmt(const RowsArgs& a, int act, hipStream_t st) {
     if (token_small_tiles(a)) return launch_token_rag<FMT, 2, 1>(a, act, st);
-    const bool narrow = a.N <= 128 || a.K <= 64;
+    const bool narrow = a.N <= 128 || (a.K <= 64 && a.N <= 512);
     if (!token_whole(a)) return narrow ? launch_token_rag<FMT, 2, 4>(a, act, st) : launch_token_rag<FMT, 4, 4>(a, act, st);
     if (narrow) launch_token_whole<FMT, 2>(a, act, st);
     else launch_token_whole<FMT, 4>(a, act, st);
