@@ -30,7 +30,7 @@ static void launch_gemm_t(const RowsArgs& a, hipStream_t st) {
 // Tile shape: 128 x 256 for large M and N (two blocks per CU); 64 x 64 while
 // there are at most two per CU (a lone block's K steps take half the time), two
 // and a half where the epilogue has integer terms; then 128 x 128, but with at
-// most one per CU (two for K <= 256) 64 x 128, which gives more blocks, where K <
+// most one per CU (one and a half for K <= 256) 64 x 128, which gives more blocks, where K <
 // 1024 or the epilogue has terms.  Measured on MI355X (us, 64 x 64 / 64 x 128 /
 // 128 x 128): codes in, int32 out, 4096 x 3072 -> 256 8.5 / 9.9 / 14.4, 12000 x
 // 1536 -> 256 (752 blocks of 64 x 64) 12.2 / 9.8 / 9.7, 9000 x 2048 -> 384 17.4 /
@@ -50,7 +50,7 @@ static int gemm_shape(const RowsArgs& a) {
     const int64_t b64 = ((a.M + 63) / 64) * ((static_cast<int64_t>(a.N) + 63) / 64);
     if (a.N <= 64 || 2 * b64 <= (terms ? 5 : 4) * cus) return 22;
     const int64_t b128 = ((a.M + 127) / 128) * ((static_cast<int64_t>(a.N) + 127) / 128);
-    return (a.K < 1024 || terms) && b128 <= (a.K <= 256 ? 2 * cus : cus) ? 24 : 44;
+    return (a.K < 1024 || terms) && 2 * b128 <= (a.K <= 256 ? 3 : 2) * cus ? 24 : 44;
 }
 
 template <int TM, int TN, int OUT, int ACT>

@@ -707,10 +707,11 @@ static bool use_skinny(const RowsArgs& a) {
 // split) over K = 192 .. 512, 22 row counts from 600 to 100000, 12 widths:
 //   K <= 256: one-pass for whole shapes (20000 x 256 -> 512 17.9 / 20.4).  The
 //     masked form loses to the GEMM at K = 256 (3000 -> 1000 15.4 / 10.8, 20000 ->
-//     300 21.9 / 18.1, 80000 -> 800 92 / 75), at K = 192 with at most three
-//     quarters of a 64-row tile per CU (6000 -> 640 13.8 / 10.5) and where the
-//     last round is half empty (40000 -> 1000 58 / 52), at K = 128 into wide rows
-//     (3000 -> 2000 15.1 / 11.8, 40000 -> 800 47 / 40);
+//     300 21.9 / 18.1, 80000 -> 800 92 / 75; not in one nearly full round of nearly
+//     full chunks, 32768 -> 500 27.4 / 29.6), below that with few 64-row tiles per
+//     CU (6000 x 192 -> 640 13.8 / 10.5, 3000 x 128 -> 2000 15.1 / 11.8; 12000 x 192
+//     -> 768 17.1 / 19.7, 12000 x 128 -> 800 15.7 / 17.6) and where a second round
+//     is half empty (40000 x 192 -> 1000 58 / 52, 40000 x 128 -> 800 47 / 40);
 //   larger K at 16-row tiles: one-pass up to 2.5 (row tile, 128-column chunk)
 //     pairs per CU (2000 x 384 -> 500 9.2 / 9.7, 3000 -> 1000 16.9 / 12.3), 3.5 with
 //     part lines at K = 512 (2500 x 512 -> 500 12.3 / 13.7, 2000 -> 1000 15.2 /
@@ -733,9 +734,16 @@ static bool split_faster(const RowsArgs& a) {
     const bool part_lines = a.N % 32 != 0;
     if (a.K <= 256) {
         if (token_whole(a)) return false;
-        if (a.K == 256) return a.N > 192 && 2 * pairs > 7 * cus;
-        if (token_small_tiles(a)) return false;
-        return a.K == 128 ? a.N >= 768 : a.N > 256 && (4 * tiles <= 3 * cus || (tiles > slots && fill < 65));
+        if (a.K == 256) {
+            const int chunks = (a.N + 255) / 256;
+            if (tiles > cus && tiles <= slots && fill >= 75 && a.N >= 192 * chunks) return false;
+            return a.N > 192 && 2 * pairs > 7 * cus;
+        }
+        if (token_small_tiles(a) || a.N <= (a.K == 128 ? 767 : 256)) return false;
+        if (a.K == 128 && a.N >= 1024) return true;
+        // Eighths of a tile per CU.
+        const int eighths = a.K == 128 || (a.N > 640 && a.N < 2048) ? 4 : a.N <= 640 ? 6 : 3;
+        return 8 * tiles <= eighths * cus || (tiles > slots && fill < 65);
     }
     if (token_small_tiles(a))
         return a.N > (a.K == 512 && !part_lines ? 255 : 384) && 2 * pairs > (a.K == 512 && part_lines ? 7 : 5) * cus;
