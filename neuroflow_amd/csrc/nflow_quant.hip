@@ -711,7 +711,8 @@ static bool use_skinny(const RowsArgs& a) {
 //     full chunks, 32768 -> 500 27.4 / 29.6), below that with few 64-row tiles per
 //     CU (6000 x 192 -> 640 13.8 / 10.5, 3000 x 128 -> 2000 15.1 / 11.8; 12000 x 192
 //     -> 768 17.1 / 19.7, 12000 x 128 -> 800 15.7 / 17.6) and where a second round
-//     is half empty (40000 x 192 -> 1000 58 / 52, 40000 x 128 -> 800 47 / 40);
+//     is half empty (40000 x 192 -> 1000 58 / 52, 40000 x 128 -> 800 47 / 40), and at
+//     K = 128 from N = 1024 on (6000 -> 2000 19.5 / 16.7; 20000 -> 2000 42 / 45);
 //   larger K at 16-row tiles: one-pass up to 2.5 (row tile, 128-column chunk)
 //     pairs per CU (2000 x 384 -> 500 9.2 / 9.7, 3000 -> 1000 16.9 / 12.3), 3.5 with
 //     part lines at K = 512 (2500 x 512 -> 500 12.3 / 13.7, 2000 -> 1000 15.2 /
